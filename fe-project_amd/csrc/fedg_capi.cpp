@@ -1232,6 +1232,12 @@ int hevi_work_get(fedg_ctx* ctx, HeviWork** w) {
   al(&h->buv, 2 * n);
   al(&h->coef, 3 * n);
   al(&h->partial, 256);
+  // line-solve scratch: 16 wavefronts per CU (twice what is resident at p = 7,
+  // so that the last ones balance), no more than the lines fill
+  const size_t lpw = m.n1 <= 4 ? 16 : 8, nline = (size_t)m.Ne2D * m.Nfp;
+  const size_t nwave = std::min(((nline + lpw - 1) / lpw + 1) / 2 * 2, (size_t)16 * ctx->ncu);
+  h->lines_n = line_list_doubles((long)((nline + lpw - 1) / lpw)) + nwave * line_scratch_per_wave(m.n1, m.Ne / m.Ne2D);
+  al(&h->lines, h->lines_n);
   ctx->hevi = h;
   if (rc != FEDG_OK) {
     hevi_work_free(ctx);
@@ -1246,7 +1252,7 @@ void hevi_work_free(fedg_ctx* ctx) {
   if (!h) return;
   for (int v = 0; v < 5; ++v)
     if (h->pv[v]) (void)hipFree(h->pv[v]);
-  double* bufs[] = {h->alph, h->b3, h->buv, h->coef, h->partial, h->r_plain, h->r_guess, h->flag};
+  double* bufs[] = {h->alph, h->b3, h->buv, h->coef, h->lines, h->partial, h->r_plain, h->r_guess, h->flag};
   for (double* b : bufs)
     if (b) (void)hipFree(b);
   if (h->X) (void)hipFree(h->X);

@@ -11,6 +11,9 @@ struct HeviWork {
   double* b3;         // (3, Np*Ne) DDENS, MOMZ, DRHOT rhs
   double* buv;        // (2, Np*Ne) MOMX, MOMY rhs
   double* coef;       // (3, Np*Ne) POT, WT, DPDRHOT
+  double* lines;      // line solves: list of groups to solve with row exchanges, then the level
+                      // solutions of the wavefronts in flight
+  size_t lines_n;     // doubles in it
   double* partial;    // 256 partial sums (residual norms)
   double partial_h[256];
   // learned initial guess (allocated on first use)
@@ -50,6 +53,16 @@ struct HeviStore {
   double* var0[5];    // or null
   double* varTmp[5];  // or null
 };
+
+// Doubles of line-solve scratch one wavefront needs: per level the 3 n1 rows
+// of up to four right-hand sides of its 64 / 4 (n1 <= 4) or 64 / 8 lines.
+inline size_t line_scratch_per_wave(int n1, int NeZ) {
+  return (size_t)NeZ * 3 * n1 * 4 * (n1 <= 4 ? 16 : 8);
+}
+
+// Doubles (a multiple of 32) of the list that precedes it: a count and up to
+// ngroup group numbers.
+inline size_t line_list_doubles(long ngroup) { return ((size_t)ngroup / 2 + 1 + 31) / 32 * 32; }
 
 int hevi_work_get(fedg_ctx* ctx, HeviWork** w);
 void hevi_work_free(fedg_ctx* ctx);

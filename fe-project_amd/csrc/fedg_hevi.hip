@@ -6,27 +6,28 @@
 //   1. hevi_rhs_uv   (element, one thread per node): the damping coefficient
 //      alph at every vertical face node from q^n, the horizontal-momentum
 //      face jumps of the iterate, their lift, MOMX_t / MOMY_t and the uv rhs;
-//   2. hevi_solve_uv (64/8 lines per wavefront, a lane per block row):
+//   2. hevi_solve_uv (64/8 lines per wavefront at p = 7, a lane per node):
 //      assembles the N x N blocks of construct_matbnd_uv level by level,
 //      block-Thomas elimination with the pivoted LU of solve_NnodeN_uv, back
 //      substitution, MOMX, MOMY += increment;
 //   3. hevi_rhs3     (element): vertical fluxes of DDENS, MOMZ, DRHOT, their
 //      face jumps, Dz and lift, VFilterPM1 buoyancy, the var3 rhs and the
 //      linearisation coefficients POT, WT, DPDRHOT;
-//   4. hevi_solve3   (two lines per wavefront at p = 7, a lane per block
-//      row): the 3N x 3N blocks of construct_matbnd, block-Thomas with the LU
-//      of solve_NnodeN_var3, DDENS, MOMZ, DRHOT += increment.
+//   4. hevi_solve3   (eight lines per wavefront at p = 7, a lane per node):
+//      the 3N x 3N blocks of construct_matbnd, block-Thomas with the LU of
+//      solve_NnodeN_var3, DDENS, MOMZ, DRHOT += increment.
 // A line is the column of one horizontal node (ij) of one horizontal element
 // through all NeZ elements; everything the implicit operator couples lies on
-// it.  A block's rows stay in registers of their lanes; pivoting exchanges
-// row positions, the pivot row and the solved entries travel by cross-lane
-// shuffles, and the levels' solutions wait in LDS for the block back
-// substitution.  Every entry sees the same operations in the same order as
-// the reference's serial loops, so results are bit for bit those of the CPU
-// restatement.
+// it.  A block's columns stay in registers of their lanes, multipliers travel
+// by cross-lane moves, and the levels' solutions wait in a scratch area for the
+// block back substitution.  Every entry sees the same operations in the same
+// order as the reference's serial loops, so results are bit for bit those of
+// the CPU restatement.
+#include <algorithm>
 #include <cfloat>
 #include <cmath>
 #include <mutex>
+#include <type_traits>
 
 #include "fedg_device.h"
 #include "fedg_hevi.h"
@@ -55,6 +56,8 @@ struct HeviArgs {
   double* buv;             // (2, Np*Ne)
   double* coef;            // (3, Np*Ne): POT, WT, DPDRHOT
   double* T[5];            // implicit-operator tendencies (VID order), written when want_T
+  int* flagged;            // groups of lines whose pivots leave the diagonal: their number, then the groups
+  double* lines;           // scratch of the line solves: the level solutions of every wavefront in flight
   double impl_fac;
   int want_b;              // form the rhs (Newton) or only the operator (impl_fac = 0)
   int NeZ;
@@ -100,6 +103,7 @@ __device__ __forceinline__ void hevi_rhs_uv_body(const HeviArgs& a) {
   const DevMesh& m = a.m;
   const Consts& c = a.c;
   const uint32_t o = (uint32_t)Np * ke + p;
+  if (a.flagged && ke == 0 && p == 0) a.flagged[0] = 0;  // for the line solve that follows
   const double gamm = c.CPdry / c.CVdry, rgamm = c.CVdry / c.CPdry;
   const double PRES0ovRdry = c.PRES00 / c.Rdry, rP0 = 1.0 / c.PRES00;
   if (!a.alph_ready) {
@@ -286,418 +290,653 @@ __device__ __forceinline__ void hevi_rhs3_body(const HeviArgs& a) {
 }
 
 // ---------------------------------------------------------------------------
-// Wavefront-cooperative pivoted LU + solve of solve_NnodeN_var3 / _uv
-// (FDS/scale_atm_dyn_dgm_hevi_common_linalgebra.F90:2142-2445) for an n x n
-// block (rows in the lanes' registers) and NR right-hand sides (solution to
-// LDS).
-// ---------------------------------------------------------------------------
-// Line solves.  A wavefront holds 64/SEG lines, one per segment of SEG lanes;
-// lane r of a segment owns row r of the level's n x n block in registers and
-// the rows' right-hand-side entries.  Partial pivoting moves rows by
-// exchanging their positions (pos), not their data: the operations every
-// entry sees -- pivot choice, reciprocal of the pivot, scaling of the column,
-// rank-1 update, forward substitution by columns, back substitution in
-// ascending column order -- are those of the reference's serial loops
-// (FDS/scale_atm_dyn_dgm_hevi_common_linalgebra.F90:2142-2445), so results
-// are bit for bit the CPU restatement's (rows outside the update subtract an
-// exact zero, which can only turn a -0 entry into +0).
+// Line solves: block Thomas over the levels of a vertical line, each level's
+// n x n block (n = NS N, unknown j = NS node + variable) by the pivoted LU of
+// solve_NnodeN_var3 / _uv (FDS/scale_atm_dyn_dgm_hevi_common_linalgebra.F90:
+// 2142-2445).
+//
+// A line owns a segment of SEG lanes (4 for N <= 4, else 8): lane c holds the
+// NS columns of node c, A[s][i] = entry (row i, column NS c + s), and lanes
+// 0..3 hold up to four right-hand sides in B[i]; 64 / SEG lines share a
+// wavefront.  With whole columns in a lane's registers
+//  - the pivot search, the reciprocal and the scaled column are lane-local;
+//    only the multipliers l(i) travel, from a lane known at compile time
+//    (DPP broadcasts: no LDS traffic in the elimination);
+//  - one broadcast l(i) updates row i of all NS columns and the right-hand
+//    sides of every line of the wavefront;
+//  - rows are exchanged in the registers, only when a line's pivot is not on
+//    the diagonal (rare for the diagonally dominant blocks of the usual steps).
+// Bound: FP64 VALU issue (about 5,700 instructions per level of eight p = 7
+// lines, 11 per multiplier: product, two moves, four multiply-subtract pairs;
+// VALU busy 0.78 of the time).  A block needs 2 n (NS + 1) VGPRs (192 at
+// p = 7), so two wavefronts share a SIMD and nothing else may stay in
+// registers across the LU: a spilled address waits, in the one order vector
+// memory completes in, for the stores before it (with 40 spilled registers
+// 3.5 ms, with 300 6.9 ms).  The levels' solutions (b and the coupling
+// columns) go to a scratch area of the wavefront's own, whose traffic hides
+// behind the arithmetic, and a level's operands are loaded during the level
+// before.
+// Measured on the 240 x 16 x 8 p = 7 channel, per solve: 12.6 ms in the layout
+// before (one row per lane, two lines per wavefront, the pivot row through LDS
+// permutes) -> 3.2 ms; uv 0.745 -> 0.555 ms; 12 x 6 x 6 p = 3: 56 -> 37 us, uv
+// 17.1 -> 12.7 us.
+// The operations every entry sees -- pivot choice (first largest), reciprocal
+// of the pivot, scaling of the column, rank-1 update, forward substitution,
+// back substitution in ascending column order -- are those of the reference's
+// serial loops, so results are bit for bit the CPU restatement's.
 
-// Cross-lane exchanges inside a segment: DPP permutations within 16-lane
-// rows, ds_swizzle between the two rows of a 32-lane segment (every DPP
-// control used here reads a valid lane, so no lane keeps an old value).
-template <int CTRL>
-__device__ __forceinline__ int dpp_i(int v) {
-  return __builtin_amdgcn_mov_dpp(v, CTRL, 0xF, 0xF, true);
-}
-
-// maximum over the segment of a double that is never NaN
-template <int CTRL>
-__device__ __forceinline__ double dpp_d(double v) {
-  return __hiloint2double(dpp_i<CTRL>(__double2hiint(v)), dpp_i<CTRL>(__double2loint(v)));
-}
-// v_max_f64: the values reduced are |A(i,k)| (never -0), the sentinels -1
-// and -2 and +inf, never NaN, so the maximum is the one of b > a ? b : a
-// bit for bit, in one instruction instead of a compare and two selects
-__device__ __forceinline__ double dmax(double a, double b) { return __builtin_fmax(a, b); }
-template <int SEG>
-__device__ __forceinline__ double seg_max(double v) {
-  v = dmax(v, dpp_d<0xB1>(v));
-  v = dmax(v, dpp_d<0x4E>(v));
-  v = dmax(v, dpp_d<0x141>(v));
-  if constexpr (SEG >= 16) v = dmax(v, dpp_d<0x140>(v));
-  if constexpr (SEG >= 32) {
-    constexpr int X16 = (0x10 << 10) | 0x1F;
-    v = dmax(v, __hiloint2double(__builtin_amdgcn_ds_swizzle(__double2hiint(v), X16),
-                                 __builtin_amdgcn_ds_swizzle(__double2loint(v), X16)));
+template <int I, int E, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (I < E) {
+    f(std::integral_constant<int, I>{});
+    static_for<I + 1, E>(f);
   }
-  if constexpr (SEG >= 64) v = dmax(v, __shfl_xor(v, 32, 64));
-  return v;
 }
-template <int SEG>
-__device__ __forceinline__ int seg_min_i(int v) {
-  v = min(v, dpp_i<0xB1>(v));
-  v = min(v, dpp_i<0x4E>(v));
-  v = min(v, dpp_i<0x141>(v));
-  if constexpr (SEG >= 16) v = min(v, dpp_i<0x140>(v));
-  if constexpr (SEG >= 32) v = min(v, __builtin_amdgcn_ds_swizzle(v, (0x10 << 10) | 0x1F));
-  if constexpr (SEG >= 64) v = min(v, __shfl_xor(v, 32, 64));
-  return v;
-}
-// lowest lane of the segment whose predicate is set (the predicate holds for
-// at least one lane of every segment); *several: more than one lane holds it
-template <int SEG>
-__device__ __forceinline__ int seg_first(bool pred, bool* several) {
-  const unsigned long long bal = __ballot(pred);
-  const int sb = threadIdx.x & ~(SEG - 1);
-  if constexpr (SEG == 64) {
-    *several = __popcll(bal) > 1;
-    return __builtin_ctzll(bal);
+
+// the value of lane C of the caller's SEG-lane segment, in two steps: for 8
+// lanes row_newbcast of lane C to the 16-lane row, then of lane C + 8 to its
+// upper half (banks 2 and 3); for 4 lanes quad_perm [C, C, C, C]
+template <int SEG, int C>
+__device__ __forceinline__ double bcast_1(double v) {
+  if constexpr (SEG == 4) {
+    constexpr int q = C * 0x55;
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), q, 0xF, 0xF, true),
+                            __builtin_amdgcn_mov_dpp(__double2loint(v), q, 0xF, 0xF, true));
   } else {
-    const unsigned s = (unsigned)(bal >> sb) & (unsigned)((1ull << SEG) - 1);
-    *several = __popc(s) > 1;
-    return sb + __builtin_ctz(s);
+    return __longlong_as_double(__builtin_amdgcn_mov_dpp(__double_as_longlong(v), 0x150 + C, 0xF, 0xF, true));
+  }
+}
+template <int SEG, int C>
+__device__ __forceinline__ double bcast_2(double r, double v) {
+  if constexpr (SEG == 4) return r;
+  else
+    return __longlong_as_double(__builtin_amdgcn_update_dpp(__double_as_longlong(r), __double_as_longlong(v),
+                                                            0x158 + C, 0xF, 0xC, false));
+}
+template <int SEG, int C>
+__device__ __forceinline__ double bcast(double v) {
+  return bcast_2<SEG, C>(bcast_1<SEG, C>(v), v);
+}
+// the values are formed here, in this order (no instruction)
+template <int M>
+__device__ __forceinline__ void pin(double* x) {
+  if constexpr (M == 1) asm volatile("" : "+v"(x[0]));
+  if constexpr (M == 2) asm volatile("" : "+v"(x[0]), "+v"(x[1]));
+  if constexpr (M == 3) asm volatile("" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]));
+  if constexpr (M == 4) asm volatile("" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]));
+}
+template <int SEG, int C>
+__device__ __forceinline__ int bcast_i(int v) {
+  if constexpr (SEG == 4) {
+    return __builtin_amdgcn_mov_dpp(v, C * 0x55, 0xF, 0xF, true);
+  } else {
+    const int r = __builtin_amdgcn_mov_dpp(v, 0x150 + C, 0xF, 0xF, true);
+    return __builtin_amdgcn_update_dpp(r, v, 0x158 + C, 0xF, 0xC, false);
   }
 }
 
-// LU with partial pivoting of the segment's n x n block (row r in A of lane
-// r), applied to NR right-hand sides as it goes (x[q] of lane r: entry r of
-// rhs q; the row operations on them are the forward substitution), then back
-// substitution.  Rows are never moved: a row's position (pos) changes when
-// it is swapped with the pivot row, and the pivot row and the entries solved
-// travel by cross-lane permutes or LDS.  Every lane of the single-wavefront
-// workgroup calls it.
-//  - the pivot search reduces |A(i,k)| alone and finds the row by a ballot;
-//    only when several rows hold the maximum does a second reduction pick
-//    the first position among them;
-//  - every lane forms 1 / A(i,k) before the search, and the pivot lane's
-//    reciprocal is the one broadcast;
-//  - all NR right-hand sides are carried (unused ones hold zeros);
-//  - after the elimination each row lane stores its row of U (the reciprocal
-//    of the pivot on the diagonal) in the segment's triangular LDS block U
-//    (row i at i n - i (i - 1) / 2), and the back substitution runs on the NR
-//    right-hand-side lanes alone, reading U from LDS.
-// X (LDS, column-major n x NR) receives the solution.  U holds
-// n (n + 1) / 2 + SEG doubles (the last SEG are write sinks).
-template <int n, int SEG, int NR>
-__device__ __forceinline__ void lu_solve_tri(double (&A)[n], double (&x)[NR], bool act, double* U, double* X) {
-  const int lane = threadIdx.x;
-  int pos = act ? (lane % SEG) : (1 << 20);
+// LDS of one wavefront: writes by some lanes are read by others of the same
+// wavefront, whose LDS operations complete in order; only the compiler has to
+// keep the order.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// exchanges two register pairs where they are
+__device__ __forceinline__ void swap_in_place(double& x, double& y) {
+  double t;
+  asm("v_mov_b64 %2, %0\n\tv_mov_b64 %0, %1\n\tv_mov_b64 %1, %2" : "+v"(x), "+v"(y), "=&v"(t));
+}
+
+// row i of the block is complete here (no instruction)
+template <int NS, int n>
+__device__ __forceinline__ void keep_order(double (&A)[NS][n], double (&B)[n], int i) {
+  if constexpr (NS == 1) asm volatile("" : "+v"(A[0][i]), "+v"(B[i]));
+  else asm volatile("" : "+v"(A[0][i]), "+v"(A[1][i]), "+v"(A[2][i]), "+v"(B[i]));
+}
+
+// LU of every segment's block, applied to the right-hand sides as it goes,
+// then back substitution: B becomes the solution (lanes 0..3).
+// PIVOT false: no rows are exchanged; false is returned when a line's pivot
+// was not on the diagonal (its result is then to be discarded), so that the
+// usual path is one stretch of code without a branch, whose registers hold
+// the blocks.  PIVOT true: rows are exchanged in the registers (the branches
+// make the allocator spill).
+// ahead() is called in the back substitution once registers have come free:
+// the next level's loads, whose latency the rest of it covers.
+template <int NS, int N, int SEG, bool PIVOT, class F>
+__device__ __forceinline__ bool lu_solve_cols(double (&A)[NS][NS * N], double (&B)[NS * N], int c, F&& ahead) {
+  constexpr int n = NS * N;
+  double inv = 1.0 / A[0][0];
+  unsigned long long off = 0;
+  static_for<0, n>([&](auto K) __attribute__((always_inline)) {
+    constexpr int k = decltype(K)::value, ck = k / NS, sk = k % NS;
+    if constexpr (k < n - 1) {
+      bool larger = false;
 #pragma unroll
-  for (int k = 0; k < n; ++k) {
-    const double inv = 1.0 / A[k];
-    const bool elig = act && pos >= k;
-    double av = -2.0;
-    if (elig) {
-      const double t = fabs(A[k]);
-      av = (t == t) ? t : (pos == k ? __builtin_huge_val() : -1.0);
+      for (int i = k + 1; i < n; ++i) larger = larger | (fabs(A[sk][i]) > fabs(A[sk][k]));
+      const unsigned long long here = __ballot(larger & (c == ck));
+      if constexpr (!PIVOT) {
+        off |= here;
+        asm volatile("" : "+s"(off));  // compared now: the column's old entries are not kept for later
+      } else if (here) {
+        int p = k;
+        double big = fabs(A[sk][k]);
+#pragma unroll
+        for (int i = k + 1; i < n; ++i) {
+          const double t = fabs(A[sk][i]);
+          if (t > big) {
+            big = t;
+            p = i;
+          }
+        }
+        p = bcast_i<SEG, ck>(p);
+#pragma unroll
+        for (int i = k + 1; i < n; ++i) {
+          if (p == i) {
+#pragma unroll
+            for (int s = 0; s < NS; ++s) swap_in_place(A[s][i], A[s][k]);
+            swap_in_place(B[i], B[k]);
+          }
+        }
+        inv = 1.0 / A[sk][k];
+      }
     }
-    const double mx = seg_max<SEG>(av);
-    bool several;
-    int lp = seg_first<SEG>(av == mx, &several);
-    if (__any(several)) {
-      const int first = seg_min_i<SEG>(av == mx ? pos : (1 << 30));
-      lp = seg_first<SEG>(av == mx && pos == first, &several);
+    const double inv_k = inv;
+    // Rows in chunks of CH, the multipliers one chunk ahead: each step of a
+    // chunk's broadcasts lies more than the two instructions a DPP operand
+    // needs behind the step before it, and no more multipliers are held than
+    // the registers take.
+    constexpr int CH = 3;
+    auto multipliers = [&](auto I0, double* l) __attribute__((always_inline)) {
+      constexpr int i0 = decltype(I0)::value, M = n - i0 < CH ? n - i0 : CH;
+      if constexpr (M > 0) {
+        double x[M];
+#pragma unroll
+        for (int r = 0; r < M; ++r) x[r] = A[sk][i0 + r] * inv_k;
+        pin<M>(x);
+#pragma unroll
+        for (int r = 0; r < M; ++r) l[r] = bcast_1<SEG, ck>(x[r]);
+        pin<M>(l);
+#pragma unroll
+        for (int r = 0; r < M; ++r) l[r] = bcast_2<SEG, ck>(l[r], x[r]);
+        pin<M>(l);
+      }
+    };
+    double l[CH] = {}, lnext[CH] = {};
+    multipliers(std::integral_constant<int, k + 1>{}, l);
+    static_for<0, (n - 1 - k + CH - 1) / CH>([&](auto Q) __attribute__((always_inline)) {
+      constexpr int i0 = k + 1 + decltype(Q)::value * CH, M = n - i0 < CH ? n - i0 : CH;
+      __builtin_amdgcn_sched_barrier(0);
+      multipliers(std::integral_constant<int, i0 + CH>{}, lnext);
+#pragma unroll
+      for (int r = 0; r < M; ++r) {
+        const int i = i0 + r;
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+          if (NS * (N - 1) + s > k) A[s][i] = A[s][i] - l[r] * A[s][k];  // some lane's column is still ahead
+        B[i] = B[i] - B[k] * l[r];
+        keep_order(A, B, i);
+        if (i == k + 1) inv = 1.0 / A[(k + 1) % NS][i];
+      }
+#pragma unroll
+      for (int r = 0; r < CH; ++r) l[r] = lnext[r];
+    });
+    // the reciprocal of the pivot on the diagonal of U
+    A[sk][k] = (c == ck) ? inv_k : A[sk][k];
+  });
+  static_for<0, n>([&](auto I) __attribute__((always_inline)) {
+    constexpr int i = n - 1 - decltype(I)::value;
+    // row i's broadcasts start no earlier than row i + 2 is done (all of them
+    // hoisted to the top would not fit the registers)
+    if constexpr (i + 2 < n) {
+#pragma unroll
+      for (int s = 0; s < NS; ++s) asm volatile("" : "+v"(A[s][i]), "+v"(B[i + 2]));
     }
-    const bool isp = lane == lp;
-    const bool below = elig && !isp;
-    const double dinv = __shfl(inv, lp, 64);
-    const double l = A[k] * dinv;
-    const double l0 = below ? l : 0.0;
-#pragma unroll
-    for (int j = k + 1; j < n; ++j) {
-      const double pj = __shfl(A[j], lp, 64);
-      A[j] = A[j] - l0 * pj;
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (i == n - 1 - n / 3) {
+      ahead();
+      __builtin_amdgcn_sched_barrier(0);
     }
+    double t = B[i];
+    const double d = bcast<SEG, i / NS>(A[i % NS][i]);
+    constexpr int CB = 4;
+    static_for<0, (n - 1 - i + CB - 1) / CB>([&](auto Q) __attribute__((always_inline)) {
+      constexpr int j0 = i + 1 + decltype(Q)::value * CB, M = n - j0 < CB ? n - j0 : CB;
+      double x[M];
+      static_for<0, M>([&](auto R) __attribute__((always_inline)) {
+        constexpr int j = j0 + decltype(R)::value;
+        x[j - j0] = bcast_1<SEG, j / NS>(A[j % NS][i]);
+      });
+      pin<M>(x);
+      static_for<0, M>([&](auto R) __attribute__((always_inline)) {
+        constexpr int j = j0 + decltype(R)::value;
+        x[j - j0] = bcast_2<SEG, j / NS>(x[j - j0], A[j % NS][i]) * B[j];
+      });
+      pin<M>(x);
 #pragma unroll
-    for (int q = 0; q < NR; ++q) {
-      const double pq = __shfl(x[q], lp, 64);
-      x[q] = x[q] - pq * l0;
-    }
-    const int ppos = __shfl(pos, lp, 64);
-    if (act) {
-      if (pos == k) pos = ppos;
-      else if (isp) pos = k;
-    }
-    if (isp) A[k] = dinv;
-    else if (below) A[k] = l;
-  }
-  // rows of U and the forward-reduced right-hand sides to LDS
-  constexpr int nt = n * (n + 1) / 2;
-  const int sink = nt + lane % SEG;
-  const int base = act ? pos * n - pos * (pos - 1) / 2 - pos : 0;
-#pragma unroll
-  for (int j = 0; j < n; ++j) U[(act && j >= pos) ? base + j : sink] = A[j];
-  if (act) {
-#pragma unroll
-    for (int q = 0; q < NR; ++q) X[pos + n * q] = x[q];
-  }
-  __syncthreads();
-  // back substitution on the right-hand-side lanes, each row's sum in
-  // ascending column order
-  const int rq = lane % SEG;
-  if (rq < NR) {
-    double* Xq = X + n * rq;
-#pragma unroll
-    for (int i = n - 1; i >= 0; --i) {
-      const double* Ui = U + (i * n - i * (i - 1) / 2 - i);
-      double t = Xq[i];
-#pragma unroll
-      for (int j = i + 1; j < n; ++j) t = t - Ui[j] * Xq[j];
-      Xq[i] = t * Ui[i];
-    }
-  }
-  __syncthreads();
+      for (int r = 0; r < M; ++r) t = t - x[r];
+    });
+    B[i] = t * d;
+  });
+  return off == 0;
 }
 
 template <int N1>
 struct LineSeg {
-  static constexpr int n3 = 3 * N1;
-  static constexpr int SEG3 = n3 <= 8 ? 8 : (n3 <= 16 ? 16 : (n3 <= 32 ? 32 : 64));
-  static constexpr int SEGU = N1 <= 8 ? 8 : (N1 <= 16 ? 16 : 32);
+  static constexpr int SEG = N1 <= 4 ? 4 : 8;
+  static constexpr int LPW = 64 / SEG;  // lines per wavefront
+  static constexpr int WPB = 2;         // wavefronts per workgroup: adjacent lines share 128-byte memory lines
 };
+
+// What lane c loads of a line's level kz for its node (ij, c): the metric
+// and, for the bottom (f = 0) and top (f = 1) face, Lift, Fscale, the damping
+// coefficients of both sides and nz.
+struct LineNode {
+  double G, GH, Lift[2], Fs[2], am[2], ap[2], nz[2];
+};
+// em: EMap3Dto2D of the level's element, loaded a level earlier
+template <int N>
+__device__ __forceinline__ void load_node(const HeviArgs& a, int ke2D, int ij, int kz, int pv, int em, bool with_nz,
+                                          LineNode& L) {
+  constexpr int Nfp = N * N, Np = N * N * N;
+  const DevMesh& m = a.m;
+  const int NeZ = a.NeZ, ke = ke2D + kz * m.Ne2D;
+  L.G = ldg(m.Gsqrt, (uint32_t)(Np * ke + ij + Nfp * pv));
+  L.GH = ldg(m.GsqrtH, (uint32_t)(ij + Nfp * em));
+#pragma unroll
+  for (int f = 0; f < 2; ++f) {
+    const bool bc = f == 0 ? kz == 0 : kz == NeZ - 1;
+    const int ke2 = bc ? ke : (f == 0 ? ke - m.Ne2D : ke + m.Ne2D), f2 = bc ? f : 1 - f;
+    const uint32_t gfp = (uint32_t)((4 + f) * Nfp + ij) + (uint32_t)(6 * Nfp) * ke;
+    L.Lift[f] = ldg(m.Lift, (uint32_t)(ij + Nfp * pv + (4 + f) * Np));
+    L.Fs[f] = ldg(m.Fscale, gfp);
+    L.am[f] = ldg(a.alph, (uint32_t)(f * Nfp + ij) + (uint32_t)(2 * Nfp) * ke);
+    L.ap[f] = ldg(a.alph, (uint32_t)(f2 * Nfp + ij) + (uint32_t)(2 * Nfp) * ke2);
+    L.nz[f] = with_nz ? ldg(m.nz, gfp) : 0.0;
+  }
+}
+// A copy of x the compiler knows nothing about: what is derived from it is
+// formed where it is used, not kept in registers (or spilled) across the LU.
+__device__ __forceinline__ int opaque(int x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+// t1 = 0.5 impl_fac / GsqrtV Lift Fscale alph, t2 = ... nz of face f; both
+// doubled at a closed boundary (the form the boundary terms take)
+__device__ __forceinline__ double2 face_terms(const HeviArgs& a, const LineNode& L, int f, int kz) {
+  const bool bc = f == 0 ? kz == 0 : kz == a.NeZ - 1;
+  const double fac = 0.5 * a.impl_fac / (L.G / L.GH) * L.Lift[f] * L.Fs[f];
+  double2 t{fac * (L.am[f] > L.ap[f] ? L.am[f] : L.ap[f]), fac * L.nz[f]};
+  if (bc) {
+    t.x = 2.0 * t.x;
+    t.y = 2.0 * t.y;
+  }
+  return t;
+}
 
 // ---------------------------------------------------------------------------
 // 2. construct_matbnd_uv (:905-1011) + solve_uv (:589-689)
 template <int N1>
-__global__ void __launch_bounds__(64) hevi_solve_uv_kernel(const HeviArgs a) {
+__global__ void __launch_bounds__(64 * LineSeg<N1>::WPB) hevi_solve_uv_kernel(const HeviArgs a) {
   constexpr int N = N1, Nfp = N1 * N1, Np = N1 * N1 * N1;
-  constexpr int SEG = LineSeg<N1>::SEGU, LPW = 64 / SEG;
-  extern __shared__ double lds[];
-  const int lane = threadIdx.x, sg = lane / SEG, r = lane % SEG;
-  const bool act = r < N;
+  constexpr int SEG = LineSeg<N1>::SEG, LPW = LineSeg<N1>::LPW, WPB = LineSeg<N1>::WPB;
+  __shared__ double sT[WPB][LPW][2][SEG];  // face terms of the rows
+  __shared__ double sB[WPB][LPW][2][SEG];  // right-hand sides
+  __shared__ double sG[WPB][LPW][4];       // top-node solution of the level below
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, sg = lane / SEG, c = lane % SEG;
   const DevMesh& m = a.m;
-  const int nline = m.Ne2D * Nfp;
+  const int nline = m.Ne2D * Nfp, ngroup = (nline + LPW - 1) / LPW;
   const int NeZ = a.NeZ;
   const uint32_t nn = (uint32_t)Np * m.Ne;
-  constexpr int nU = N * (N + 1) / 2 + SEG;
-  double* U = lds + (size_t)sg * (nU + (size_t)NeZ * 3 * N);  // the block's U rows (triangular)
-  double* X = U + nU;  // per level: b(:,1), b(:,2), G
-  const int pv = act ? r : 0;
-  for (int g = blockIdx.x; g * LPW < nline; g += gridDim.x) {
-    const int line = g * LPW + sg;
-    const bool lv = line < nline;
-    const int ke2D = lv ? line / Nfp : 0, ij = lv ? line % Nfp : 0;
+  const int slot = blockIdx.x * WPB + w;
+  double* scr = a.lines + (size_t)slot * NeZ * N * (4 * LPW);  // [level][row][line][b1, b2, G, -]
+  const int pv = c < N ? c : N - 1;
+  double(*T)[SEG] = sT[w][sg];
+  double(*Bs)[SEG] = sB[w][sg];
+  double* G = sG[w][sg];
+  for (int g = slot; g < ngroup; g += gridDim.x * WPB) {
+    const bool lv = g * LPW + sg < nline;
+    const int line = lv ? g * LPW + sg : nline - 1;
+    const int ke2D = line / Nfp, ij = line % Nfp;
+    double B[N];
+    LineNode L;
+    double b0, b1;
+    int em = m.EMap3Dto2D[ke2D];
+    auto load = [&](int kz) __attribute__((always_inline)) {
+      const uint32_t q = (uint32_t)Np * (ke2D + kz * m.Ne2D) + ij + Nfp * pv;
+      load_node<N>(a, ke2D, ij, kz, pv, em, false, L);
+      em = m.EMap3Dto2D[ke2D + (kz + 1 < NeZ ? kz + 1 : kz) * m.Ne2D];
+      b0 = ldg(a.buv, q);
+      b1 = ldg(a.buv, q + nn);
+    };
+    load(0);
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // as in the var3 solve below
     for (int kz = 0; kz < NeZ; ++kz) {
-      const int ke = ke2D + kz * m.Ne2D;
-      double A[N];
+      T[0][c] = face_terms(a, L, 0, kz).x;
+      T[1][c] = face_terms(a, L, 1, kz).x;
+      Bs[0][c] = b0;
+      Bs[1][c] = b1;
+      if (kz > 0 && c < 3) G[c] = B[N - 1];
+      wave_sync();
+      double A[1][N];
 #pragma unroll
-      for (int c = 0; c < N; ++c) A[c] = (c == pv) ? 1.0 : 0.0;
-      double x[3] = {0.0, 0.0, 0.0};
-      double lvv = 0.0;
-      if (lv && act) {
-        const uint32_t q = (uint32_t)Np * ke + ij + Nfp * pv;
-        x[0] = ldg(a.buv, q);
-        x[1] = ldg(a.buv, q + nn);
-        // face damping of the row: f1 = 1 couples to the level below, 2 above
+      for (int i = 0; i < N; ++i) A[0][i] = (i == c) ? 1.0 : 0.0;
+      if (c == 0 && kz > 0) {
+        const double g2 = G[2];
 #pragma unroll
-        for (int f1 = 1; f1 <= 2; ++f1) {
-          const int kz2 = (f1 == 1) ? (kz - 1 > 0 ? kz - 1 : 0) : (kz + 1 < NeZ - 1 ? kz + 1 : NeZ - 1);
-          const int f2 = (f1 == 1) ? 2 : 1;
-          const bool bc = (kz == 0 && f1 == 1) || (kz == NeZ - 1 && f1 == 2);
-          if (bc) continue;
-          const int ke_2 = ke2D + kz2 * m.Ne2D;
-          const int p = ij + Nfp * pv;
-          const uint32_t gfp = (uint32_t)((3 + f1) * Nfp + ij) + (uint32_t)(6 * Nfp) * ke;
-          const double fac = 0.5 * a.impl_fac / gsqrtv(a, ke, p, N1);
-          const double am = ldg(a.alph, (uint32_t)((f1 - 1) * Nfp + ij) + (uint32_t)(2 * Nfp) * ke);
-          const double ap = ldg(a.alph, (uint32_t)((f2 - 1) * Nfp + ij) + (uint32_t)(2 * Nfp) * ke_2);
-          const double t = fac * ldg(m.Lift, (uint32_t)(p + (3 + f1) * Np)) * ldg(m.Fscale, gfp) * (am > ap ? am : ap);
-          if (f1 == 1) {
-            A[0] = A[0] + t;
-            lvv = -t;
-          } else {
-            A[N - 1] = A[N - 1] + t;
-            x[2] = -t;  // U lands in the G slot
-          }
+        for (int i = 0; i < N; ++i) A[0][i] = A[0][i] + T[0][i];
+#pragma unroll
+        for (int i = 0; i < N; ++i) A[0][i] = A[0][i] - (-T[0][i]) * g2;
+      }
+      if (c == N - 1 && kz < NeZ - 1) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) A[0][i] = A[0][i] + T[1][i];
+      }
+#pragma unroll
+      for (int i = 0; i < N; ++i) B[i] = 0.0;
+      if (c < 2) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) B[i] = Bs[c][i];
+        if (kz > 0) {
+          const double gb = G[c];
+#pragma unroll
+          for (int i = 0; i < N; ++i) B[i] = B[i] - (-T[0][i]) * gb;
         }
+      } else if (c == 2 && kz < NeZ - 1) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) B[i] = -T[1][i];
       }
-      if (kz > 0) {
-        const double* Xp = X + (size_t)(kz - 1) * 3 * N;
-        A[0] = A[0] - lvv * Xp[(N - 1) + 2 * N];
-        x[0] = x[0] - lvv * Xp[N - 1];
-        x[1] = x[1] - lvv * Xp[(N - 1) + N];
+      wave_sync();
+      (void)lu_solve_cols<1, N, SEG, true>(A, B, c, [&]() __attribute__((always_inline)) {
+        load(kz + 1 < NeZ ? kz + 1 : kz);
+      });
+      if (c < 4) {
+        double* x = scr + (size_t)kz * N * (4 * LPW) + sg * 4 + c;
+#pragma unroll
+        for (int i = 0; i < N; ++i) x[i * (4 * LPW)] = B[i];
       }
-      // at the top level the G column is zero and its solution unused
-      lu_solve_tri<N, SEG, 3>(A, x, act, U, X + (size_t)kz * 3 * N);
     }
-    for (int kz = NeZ - 2; kz >= 0; --kz) {
-      double* Xk = X + (size_t)kz * 3 * N;
-      const double* Xn = X + (size_t)(kz + 1) * 3 * N;
-      if (act) {
-        const double tmp = Xk[r + 2 * N];
-        Xk[r] = Xk[r] - tmp * Xn[0];
-        Xk[r + N] = Xk[r + N] - tmp * Xn[N];
+    wave_sync();
+    // block back substitution: lane c takes node c
+    double u = 0.0, v = 0.0, x[3], y[2];
+    auto back = [&](int kz) __attribute__((always_inline)) {  // loads of a level, issued one level ahead
+      const double* xk = scr + (size_t)kz * N * (4 * LPW) + (size_t)pv * (4 * LPW) + sg * 4;
+      const uint32_t q = (uint32_t)Np * (ke2D + kz * m.Ne2D) + ij + Nfp * pv;
+#pragma unroll
+      for (int r = 0; r < 3; ++r) x[r] = xk[r];
+      y[0] = ldg(a.pin[VU], q);
+      y[1] = ldg(a.pin[VV], q);
+    };
+    back(NeZ - 1);
+    for (int kz = NeZ - 1; kz >= 0; --kz) {
+      const double u0 = bcast<SEG, 0>(u), v0 = bcast<SEG, 0>(v);
+      u = x[0];
+      v = x[1];
+      const double tmp = x[2], yu = y[0], yv = y[1];
+      if (kz > 0) back(kz - 1);
+      if (kz < NeZ - 1) {
+        u = u - tmp * u0;
+        v = v - tmp * v0;
       }
-      __syncthreads();
-    }
-    if (lv && act) {
-      for (int kz = 0; kz < NeZ; ++kz) {
+      if (lv && c < N) {
         const uint32_t q = (uint32_t)Np * (ke2D + kz * m.Ne2D) + ij + Nfp * pv;
-        const double* Xk = X + (size_t)kz * 3 * N;
-        stg(a.pv[VU], q, ldg(a.pin[VU], q) + Xk[pv]);
-        stg(a.pv[VV], q, ldg(a.pin[VV], q) + Xk[pv + N]);
+        stg(a.pv[VU], q, yu + u);
+        stg(a.pv[VV], q, yv + v);
       }
     }
-    __syncthreads();
+    wave_sync();
   }
 }
 
 // ---------------------------------------------------------------------------
 // 4. construct_matbnd (:693-901) + solve (:329-479).
 // Unknowns of an element: (var, pv), var fastest: DENS, MOMZ, RHOT.
+// A level is assembled in two steps: lane c forms, for the rows of node c,
+// the columns of node 0 (the ones the level below couples to), the
+// right-hand side and the coupling to the level above, and passes them
+// through LDS to the lanes that hold those columns; every lane forms the
+// other columns of its own node from the rows' metric factors.
+// MODE: SOLVE_ALL, every line with row exchanges (p <= 3, whose blocks leave
+// room for them); at p >= 4 SOLVE_DIAGONAL, which gives the groups of lines
+// whose pivots leave the diagonal up to the list a.flagged (count, then group
+// numbers), and SOLVE_FLAGGED, which solves those.
+enum { SOLVE_ALL = 0, SOLVE_DIAGONAL = 1, SOLVE_FLAGGED = 2 };
 template <int N1>
-__global__ void __launch_bounds__(64) hevi_solve3_kernel(const HeviArgs a) {
+struct LineLds {
+  static constexpr int SEG = LineSeg<N1>::SEG, NR = 3 * SEG;  // rows the segment's lanes form (3 N1 of them used)
+  double E[SEG];     // E33 / GsqrtV of the rows
+  double2 T[SEG];    // face terms (t1, t2) of the rows, top face
+  double C[3][NR];   // columns of node 0
+  double B[4][NR];   // right-hand sides: b, G1, G2, G3
+  double G[4][3];    // their top-node solutions at the level below
+};
+template <int N1, int MODE>
+__global__ void __launch_bounds__(64 * LineSeg<N1>::WPB) __attribute__((amdgpu_waves_per_eu(2)))
+hevi_solve3_kernel(const HeviArgs a) {
   constexpr int N = N1, Nfp = N1 * N1, Np = N1 * N1 * N1, n3 = 3 * N1;
-  constexpr int SEG = LineSeg<N1>::SEG3, LPW = 64 / SEG;
-  extern __shared__ double lds[];
-  const int lane = threadIdx.x, sg = lane / SEG, r = lane % SEG;
-  const bool act = r < n3;
+  constexpr int SEG = LineSeg<N1>::SEG, LPW = LineSeg<N1>::LPW, WPB = LineSeg<N1>::WPB;
+  __shared__ double sD[N][N], sI[N][N];  // impl_fac D1D and impl_fac GRAV IntrpMat, by [column node][row node]
+  __shared__ LineLds<N1> sL[WPB * LPW];
   const DevMesh& m = a.m;
   const int nline = m.Ne2D * Nfp;
+  const int ngroup = MODE == SOLVE_FLAGGED ? a.flagged[0] : (nline + LPW - 1) / LPW;
+  if (MODE == SOLVE_FLAGGED && ngroup == 0) return;
   const int NeZ = a.NeZ;
   const uint32_t nn = (uint32_t)Np * m.Ne;
   const double impl_fac = a.impl_fac;
-  constexpr int nU = n3 * (n3 + 1) / 2 + SEG;
-  double* sD = lds;      // D1D
-  double* sI = sD + N * N;  // IntrpMat_VPOrdM1_tr
-  double* cf = sI + N * N + (size_t)sg * (13 * N + nU + (size_t)NeZ * 4 * n3);  // [3 levels][POT, WT, DPDRHOT][N]
-  double* t12 = cf + 9 * N;  // [face][tmp1, tmp2][N]
-  double* U = t12 + 4 * N;   // the block's U rows (triangular)
-  double* X = U + nU;        // NeZ * 4 * n3: b, G(:,1..3) per level
-  for (int e = lane; e < N * N; e += 64) {
-    sD[e] = m.D1D[e];
-    sI[e] = m.Itr[e];
+  for (int e = threadIdx.x; e < N * N; e += 64 * WPB) {
+    sD[e / N][e % N] = impl_fac * m.D1D[e];
+    sI[e % N][e / N] = impl_fac * a.c.GRAV * m.Itr[e];
   }
-  const int pv = act ? r / 3 : 0, v = r % 3;
-  for (int g = blockIdx.x; g * LPW < nline; g += gridDim.x) {
-    const int line = g * LPW + sg;
-    const bool lv = line < nline;
-    const int ke2D = lv ? line / Nfp : 0, ij = lv ? line % Nfp : 0;
+  __syncthreads();
+  const int slot = blockIdx.x * WPB + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  double* scr = a.lines + (size_t)slot * NeZ * n3 * (4 * LPW);  // [level][row][line][b, G1, G2, G3]
+  const int c0 = threadIdx.x % SEG;
+  for (int u = slot; u < ngroup; u += gridDim.x * WPB) {
+    const int g = MODE == SOLVE_FLAGGED ? __builtin_amdgcn_readfirstlane(a.flagged[1 + u]) : u;
+    double B[n3];
+    bool off = false;
+    // the level's data, loaded during the level before
+    LineNode L;
+    double b[3], cf[3], up[3], E33;  // rhs, POT / WT / DPDRHOT of the node and of the bottom node above
+    double dn[3] = {0.0, 0.0, 0.0};  // and of the top node below
+    int em;
+    // this lane's line (lanes beyond the last one work on it and store nothing)
+    auto line_of = [&](int tid) __attribute__((always_inline)) {
+      const int line = g * LPW + (tid & 63) / SEG;
+      return line < nline ? line : nline - 1;
+    };
+    auto load = [&](int kz, bool first) __attribute__((always_inline)) {
+      const int tid = opaque(threadIdx.x), c = tid % SEG, pv = c < N ? c : N - 1;
+      const int line = line_of(tid), ke2D = line / Nfp, ij = line % Nfp, ke = ke2D + kz * m.Ne2D;
+      const uint32_t q = (uint32_t)(Np * ke + ij + Nfp * pv);
+      const uint32_t qu = kz < NeZ - 1 ? (uint32_t)(Np * (ke + m.Ne2D) + ij) : q;
+      if (first) em = m.EMap3Dto2D[ke];
+      load_node<N>(a, ke2D, ij, kz, pv, em, true, L);
+      em = m.EMap3Dto2D[kz < NeZ - 1 ? ke + m.Ne2D : ke];
+      E33 = ldg(m.E33, q);
+#pragma unroll
+      for (int v = 0; v < 3; ++v) {
+        b[v] = ldg(a.b3 + (size_t)v * nn, q);
+        cf[v] = ldg(a.coef + (size_t)v * nn, q);
+        up[v] = ldg(a.coef + (size_t)v * nn, qu);
+      }
+    };
+    load(0, true);
+    // vmcnt(0): the first level waits here, so that the wait at the top of a
+    // later level (loads, then the stores of the level's solutions) need not
+    // cover those stores
+    __builtin_amdgcn_s_waitcnt(0x0F70);
     for (int kz = 0; kz < NeZ; ++kz) {
-      const int ke = ke2D + kz * m.Ne2D;
-      __syncthreads();
-      if (lv) {
-        // POT, WT, DPDRHOT of the line in this level (slot 1) and the levels below (0) / above (2)
-        for (int e = r; e < 9 * N; e += SEG) {
-          const int lvl = e / (3 * N), rr = e % (3 * N), c = rr / N, pq = rr % N;
-          int kzz = kz + lvl - 1;
-          kzz = kzz < 0 ? 0 : (kzz > NeZ - 1 ? NeZ - 1 : kzz);
-          const uint32_t q = (uint32_t)Np * (ke2D + kzz * m.Ne2D) + ij + Nfp * pq;
-          cf[e] = ldg(a.coef, q + (uint32_t)c * nn);
-        }
-        // tmp1, tmp2 of both vertical faces
-        if (r < 2 * N) {
-          const int f1 = 1 + r / N, pq = r % N;
-          const int kz2 = (f1 == 1) ? (kz - 1 > 0 ? kz - 1 : 0) : (kz + 1 < NeZ - 1 ? kz + 1 : NeZ - 1);
-          const bool bc = (kz == 0 && f1 == 1) || (kz == NeZ - 1 && f1 == 2);
-          const int f2 = bc ? f1 : ((f1 == 1) ? 2 : 1);
-          const int ke_2 = ke2D + kz2 * m.Ne2D;
-          const int p = ij + Nfp * pq;
-          const uint32_t gfp = (uint32_t)((3 + f1) * Nfp + ij) + (uint32_t)(6 * Nfp) * ke;
-          const double Lift = ldg(m.Lift, (uint32_t)(p + (3 + f1) * Np));
-          const double fac = 0.5 * impl_fac / gsqrtv(a, ke, p, N1) * Lift * ldg(m.Fscale, gfp);
-          const double am = ldg(a.alph, (uint32_t)((f1 - 1) * Nfp + ij) + (uint32_t)(2 * Nfp) * ke);
-          const double ap = ldg(a.alph, (uint32_t)((f2 - 1) * Nfp + ij) + (uint32_t)(2 * Nfp) * ke_2);
-          t12[(f1 - 1) * 2 * N + pq] = fac * (am > ap ? am : ap);
-          t12[(f1 - 1) * 2 * N + N + pq] = fac * ldg(m.nz, gfp);
-        }
+      const bool bc1 = kz == 0, bc2 = kz == NeZ - 1;
+      const int tid = opaque(threadIdx.x), c = tid % SEG, pv = c < N ? c : N - 1;
+      LineLds<N1>& S = sL[tid / SEG];
+      const double POT = cf[0], WT = cf[1], DPD = cf[2];
+      if (!bc1 && c < 4) {
+#pragma unroll
+        for (int v = 0; v < 3; ++v) S.G[c][v] = B[n3 - 3 + v];
       }
-      __syncthreads();
-      double A[n3];
-      double x[4] = {0.0, 0.0, 0.0, 0.0};
-      double lm[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-      for (int cc = 0; cc < n3; ++cc) A[cc] = 0.0;
-      if (lv && act) {
-        const double* POT0 = cf + 3 * N;  // this level
-        const double* WT0 = POT0 + N;
-        const double* DPD0 = WT0 + N;
-        const uint32_t prow = (uint32_t)Np * ke + ij + Nfp * pv;
-        const double Eg = ldg(m.E33, prow) / gsqrtv(a, ke, ij + Nfp * pv, N1);
-        x[0] = ldg(a.b3, prow + (uint32_t)v * nn);
-        const double tm1[2] = {t12[pv], t12[2 * N + pv]};      // tmp1 of faces 1, 2
-        const double tm2[2] = {t12[N + pv], t12[3 * N + pv]};  // tmp2
-        // D block with the face terms of its first / last node column
-#pragma unroll
-        for (int cc = 0; cc < n3; ++cc) {
-          const int v2 = cc % 3, pv2 = cc / 3;
-          const double Id = (pv == pv2) ? 1.0 : 0.0;
-          const double fdz = Eg * (impl_fac * sD[pv + N * pv2]);
-          const double POT = POT0[pv2], WT = WT0[pv2], DPD = DPD0[pv2];
-          double d;
-          if (v == 0) d = (v2 == 0) ? Id : (v2 == 1 ? fdz : 0.0);
-          else if (v == 1) d = (v2 == 1) ? Id : (v2 == 0 ? impl_fac * a.c.GRAV * sI[pv2 + N * pv] : fdz * DPD);
-          else d = (v2 == 0) ? -fdz * POT * WT : (v2 == 1 ? fdz * POT : Id + fdz * WT);
-#pragma unroll
-          for (int f1 = 1; f1 <= 2; ++f1) {
-            const int pv1 = (f1 == 1) ? 0 : N - 1;
-            if (pv2 != pv1) continue;
-            const bool bc = (kz == 0 && f1 == 1) || (kz == NeZ - 1 && f1 == 2);
-            const double tmp1 = tm1[f1 - 1], tmp2 = tm2[f1 - 1];
-            if (bc) {
-              if (v == 2 && v2 == 0) d = d + 2.0 * tmp2 * POT * WT;
-              else if (v == 0 && v2 == 1) d = d - 2.0 * tmp2;
-              else if (v == 1 && v2 == 1) d = d + 2.0 * tmp1;
-              else if (v == 2 && v2 == 1) d = d - 2.0 * tmp2 * POT;
-              else if (v == 2 && v2 == 2) d = d - 2.0 * tmp2 * WT;
-            } else {
-              if (v == 0 && v2 == 0) d = d + tmp1;
-              else if (v == 2 && v2 == 0) d = d + tmp2 * POT * WT;
-              else if (v == 0 && v2 == 1) d = d - tmp2;
-              else if (v == 1 && v2 == 1) d = d + tmp1;
-              else if (v == 2 && v2 == 1) d = d - tmp2 * POT;
-              else if (v == 1 && v2 == 2) d = d - tmp2 * DPD;
-              else if (v == 2 && v2 == 2) d = d + tmp1 - tmp2 * WT;
-            }
-          }
-          A[cc] = d;
+      wave_sync();
+      {
+        const double Eg = E33 / (L.G / L.GH);
+        S.E[c] = Eg;
+        // rows of node c, columns of node 0
+        const double P0 = bcast<SEG, 0>(POT), W0 = bcast<SEG, 0>(WT), D0 = bcast<SEG, 0>(DPD);
+        const double Id = (c == 0) ? 1.0 : 0.0;
+        const double fdz = Eg * sD[0][pv];
+        const double2 t = face_terms(a, L, 0, kz);
+        double d[3][3] = {{Id, fdz, 0.0}, {sI[0][pv], Id, fdz * D0}, {-fdz * P0 * W0, fdz * P0, Id + fdz * W0}};
+        d[0][1] = d[0][1] - t.y;
+        d[1][1] = d[1][1] + t.x;
+        d[2][0] = d[2][0] + t.y * P0 * W0;
+        d[2][1] = d[2][1] - t.y * P0;
+        if (!bc1) {
+          d[0][0] = d[0][0] + t.x;
+          d[1][2] = d[1][2] - t.y * D0;
+          d[2][2] = d[2][2] + t.x;
         }
-        // L (coupling to the top node of the level below) and U (bottom node
-        // of the level above, the G right-hand sides of this level)
+        d[2][2] = d[2][2] - t.y * W0;
+        // L: coupling to the top node of the level below, eliminated with its solution
+        if (!bc1) {
 #pragma unroll
-        for (int f1 = 1; f1 <= 2; ++f1) {
-          const bool bc = (kz == 0 && f1 == 1) || (kz == NeZ - 1 && f1 == 2);
-          if (bc) continue;
-          const int pv2 = (f1 == 1) ? N - 1 : 0;
-          const double* cfo = cf + (f1 == 1 ? 0 : 6 * N);
-          const double POT = cfo[pv2], WT = cfo[N + pv2], DPD = cfo[2 * N + pv2];
-          const double tmp1 = tm1[f1 - 1], tmp2 = tm2[f1 - 1];
+          for (int v = 0; v < 3; ++v) {
+            const double l0 = (v == 0) ? -t.x : (v == 1 ? 0.0 : -t.y * dn[0] * dn[1]);
+            const double l1 = (v == 0) ? +t.y : (v == 1 ? -t.x : +t.y * dn[0]);
+            const double l2 = (v == 0) ? 0.0 : (v == 1 ? +t.y * dn[2] : -t.x + t.y * dn[1]);
 #pragma unroll
-          for (int v2 = 0; v2 < 3; ++v2) {
-            double l;
-            if (v2 == 0) l = (v == 0) ? -tmp1 : (v == 1 ? 0.0 : -tmp2 * POT * WT);
-            else if (v2 == 1) l = (v == 0) ? +tmp2 : (v == 1 ? -tmp1 : +tmp2 * POT);
-            else l = (v == 0) ? 0.0 : (v == 1 ? +tmp2 * DPD : -tmp1 + tmp2 * WT);
-            if (f1 == 1) lm[v2] = l;
-            else x[1 + v2] = l;
+            for (int s = 0; s < 3; ++s) d[v][s] = d[v][s] - l0 * S.G[1 + s][0] - l1 * S.G[1 + s][1] - l2 * S.G[1 + s][2];
+            b[v] = b[v] - l0 * S.G[0][0] - l1 * S.G[0][1] - l2 * S.G[0][2];
           }
         }
-      }
-      if (kz > 0) {
-        const double* Xp = X + (size_t)(kz - 1) * 4 * n3;
-        constexpr int p1 = 3 * (N - 1), p2 = p1 + 1, p3 = p1 + 2;
+        // U: coupling to the bottom node of the level above, the G columns (none at the top level)
+        const double2 tu = face_terms(a, L, 1, kz);
+        S.T[c] = tu;
+        const double gc[3][3] = {{-tu.x, tu.y, 0.0},
+                                 {0.0, -tu.x, tu.y * up[2]},
+                                 {-tu.y * up[0] * up[1], tu.y * up[0], -tu.x + tu.y * up[1]}};
 #pragma unroll
-        for (int c = 0; c < 3; ++c)
-          A[c] = A[c] - lm[0] * Xp[p1 + n3 * (1 + c)] - lm[1] * Xp[p2 + n3 * (1 + c)] - lm[2] * Xp[p3 + n3 * (1 + c)];
-        x[0] = x[0] - lm[0] * Xp[p1] - lm[1] * Xp[p2] - lm[2] * Xp[p3];
+        for (int v = 0; v < 3; ++v) {
+          S.B[0][3 * c + v] = b[v];
+#pragma unroll
+          for (int s = 0; s < 3; ++s) {
+            S.C[s][3 * c + v] = d[v][s];
+            S.B[1 + s][3 * c + v] = bc2 ? 0.0 : gc[v][s];
+          }
+        }
+#pragma unroll
+        for (int v = 0; v < 3; ++v) dn[v] = bcast<SEG, N - 1>(cf[v]);
       }
-      // at the top level the G columns are zero and their solution unused
-      lu_solve_tri<n3, SEG, 4>(A, x, act, U, X + (size_t)kz * 4 * n3);
-    }
-    for (int kz = NeZ - 2; kz >= 0; --kz) {
-      double* Xk = X + (size_t)kz * 4 * n3;
-      const double* Xn = X + (size_t)(kz + 1) * 4 * n3;
-      if (act) Xk[r] = Xk[r] - Xk[r + n3] * Xn[0] - Xk[r + 2 * n3] * Xn[1] - Xk[r + 3 * n3] * Xn[2];
-      __syncthreads();
-    }
-    if (lv && act) {
-      double* dst = v == 0 ? a.pv[VD] : (v == 1 ? a.pv[VW] : a.pv[VT]);
-      const double* src = v == 0 ? a.pin[VD] : (v == 1 ? a.pin[VW] : a.pin[VT]);
-      for (int kz = 0; kz < NeZ; ++kz) {
-        const uint32_t q = (uint32_t)Np * (ke2D + kz * m.Ne2D) + ij + Nfp * pv;
-        stg(dst, q, ldg(src, q) + X[(size_t)kz * 4 * n3 + r]);
+      wave_sync();
+      // the other columns
+      double A[3][n3];
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const double Id = (i == c) ? 1.0 : 0.0;
+        const double fdz = S.E[i] * sD[pv][i];
+        A[0][3 * i] = Id;
+        A[1][3 * i] = fdz;
+        A[2][3 * i] = 0.0;
+        A[0][3 * i + 1] = sI[pv][i];
+        A[1][3 * i + 1] = Id;
+        A[2][3 * i + 1] = fdz * DPD;
+        A[0][3 * i + 2] = -fdz * POT * WT;
+        A[1][3 * i + 2] = fdz * POT;
+        A[2][3 * i + 2] = Id + fdz * WT;
+      }
+      // top-face terms on the columns of the last node
+      if (c == N - 1) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+          const double2 t = S.T[i];
+          A[1][3 * i] = A[1][3 * i] - t.y;
+          A[1][3 * i + 1] = A[1][3 * i + 1] + t.x;
+          A[0][3 * i + 2] = A[0][3 * i + 2] + t.y * POT * WT;
+          A[1][3 * i + 2] = A[1][3 * i + 2] - t.y * POT;
+          if (!bc2) {
+            A[0][3 * i] = A[0][3 * i] + t.x;
+            A[2][3 * i + 1] = A[2][3 * i + 1] - t.y * DPD;
+            A[2][3 * i + 2] = A[2][3 * i + 2] + t.x;
+          }
+          A[2][3 * i + 2] = A[2][3 * i + 2] - t.y * WT;
+        }
+      }
+      if (c == 0) {
+#pragma unroll
+        for (int i = 0; i < n3; ++i) {
+#pragma unroll
+          for (int s = 0; s < 3; ++s) A[s][i] = S.C[s][i];
+        }
+      }
+      {
+        const double* Bc = S.B[c < 4 ? c : 0];  // lanes beyond the right-hand sides carry a copy nobody reads
+#pragma unroll
+        for (int i = 0; i < n3; ++i) B[i] = Bc[i];
+      }
+      wave_sync();
+      if (!lu_solve_cols<3, N, SEG, MODE != SOLVE_DIAGONAL>(
+              A, B, c0, [&]() __attribute__((always_inline)) { load(bc2 ? kz : kz + 1, false); })) {
+        off = true;
+        break;
+      }
+      {
+        const int t2 = opaque(threadIdx.x), c2 = t2 % SEG;
+        if (c2 < 4) {
+          double* x = scr + (size_t)kz * n3 * (4 * LPW);
+          const uint32_t o = (uint32_t)((t2 & 63) / SEG * 4 + c2);
+#pragma unroll
+          for (int i = 0; i < n3; ++i) stg(x, o + i * (4 * LPW), B[i]);
+        }
       }
     }
+    if (MODE == SOLVE_DIAGONAL && off) {
+      if ((threadIdx.x & 63) == 0) a.flagged[1 + atomicAdd(a.flagged, 1)] = g;
+      continue;
+    }
+    wave_sync();
+    // block back substitution: lane c takes node c
+    const int tid = opaque(threadIdx.x), c = tid % SEG, pv = c < N ? c : N - 1;
+    const bool lv = g * LPW + (tid & 63) / SEG < nline;
+    const int line = line_of(tid), ke2D = line / Nfp, ij = line % Nfp;
+    double y[3] = {0.0, 0.0, 0.0}, x[3][4], p0[3];
+    auto back = [&](int kz) __attribute__((always_inline)) {  // loads of a level, issued one level ahead
+      const double* xk = scr + (size_t)kz * n3 * (4 * LPW);
+      const uint32_t o = (uint32_t)(3 * pv * (4 * LPW) + (tid & 63) / SEG * 4);
+      const uint32_t q = (uint32_t)(Np * (ke2D + kz * m.Ne2D) + ij + Nfp * pv);
+#pragma unroll
+      for (int v = 0; v < 3; ++v)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[v][r] = ldg(xk, o + v * (4 * LPW) + r);
+      p0[0] = ldg(a.pin[VD], q);
+      p0[1] = ldg(a.pin[VW], q);
+      p0[2] = ldg(a.pin[VT], q);
+    };
+    back(NeZ - 1);
+    for (int kz = NeZ - 1; kz >= 0; --kz) {
+      double y0[3], z[3][4], o[3];
+#pragma unroll
+      for (int v = 0; v < 3; ++v) {
+        y0[v] = bcast<SEG, 0>(y[v]);
+        o[v] = p0[v];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) z[v][r] = x[v][r];
+      }
+      if (kz > 0) back(kz - 1);
+#pragma unroll
+      for (int v = 0; v < 3; ++v) {
+        y[v] = z[v][0];
+        if (kz < NeZ - 1) y[v] = y[v] - z[v][1] * y0[0] - z[v][2] * y0[1] - z[v][3] * y0[2];
+      }
+      if (lv && c < N) {
+        const uint32_t q = (uint32_t)(Np * (ke2D + kz * m.Ne2D) + ij + Nfp * pv);
+        stg(a.pv[VD], q, o[0] + y[0]);
+        stg(a.pv[VW], q, o[1] + y[1]);
+        stg(a.pv[VT], q, o[2] + y[2]);
+      }
+    }
+    wave_sync();
   }
 }
 
@@ -940,32 +1179,46 @@ void launch_rhs3(fedg_ctx* ctx, const HeviArgs& a) {
     hipLaunchKernelGGL((hevi_rhs3_kernel<N1, false>), dim3(m.Ne), dim3(N1 * N1 * N1), 0, ctx->stream, a);
 }
 
+// Columns taken: those whose levels' solutions fit a 64 KB block of one
+// wavefront in the row-per-lane layout (64 / seg lines of n (n + 1) / 2 + seg
+// entries of U, 4 n per level and 13 N1 coefficients).
 template <int N1>
-size_t lds_uv(int NeZ) {
-  constexpr int nU = N1 * (N1 + 1) / 2 + LineSeg<N1>::SEGU;
-  return sizeof(double) * (size_t)(64 / LineSeg<N1>::SEGU) * (nU + (size_t)NeZ * 3 * N1);
-}
-template <int N1>
-size_t lds_3(int NeZ) {
+bool column_fits(int NeZ) {
   constexpr int n3 = 3 * N1;
-  constexpr int nU = n3 * (n3 + 1) / 2 + LineSeg<N1>::SEG3;
-  return sizeof(double) *
-         (2 * N1 * N1 + (size_t)(64 / LineSeg<N1>::SEG3) * (13 * N1 + nU + (size_t)NeZ * 4 * n3));
+  constexpr int seg3 = n3 <= 8 ? 8 : (n3 <= 16 ? 16 : 32), segu = N1 <= 8 ? 8 : 16;
+  const size_t l3 = 2 * N1 * N1 + (size_t)(64 / seg3) * (13 * N1 + n3 * (n3 + 1) / 2 + seg3 + (size_t)NeZ * 4 * n3);
+  const size_t lu = (size_t)(64 / segu) * (N1 * (N1 + 1) / 2 + segu + (size_t)NeZ * 3 * N1);
+  return sizeof(double) * l3 <= 64 * 1024 && sizeof(double) * lu <= 64 * 1024;
 }
 
 template <int N1>
-int run_newton(fedg_ctx* ctx, HeviArgs& a, int max_it, double rtol, double* resid, double* partial,
-               double* partial_h, int* it_done, double r0_ext = 0.0) {
+int run_newton(fedg_ctx* ctx, HeviArgs& a, HeviWork* w, int max_it, double rtol, double* resid, int* it_done,
+               double r0_ext = 0.0) {
   const DevMesh& m = ctx->m;
-  const int nline = m.Ne2D * N1 * N1;
-  const int guv = (nline + 64 / LineSeg<N1>::SEGU - 1) / (64 / LineSeg<N1>::SEGU);
-  const int g3 = (nline + 64 / LineSeg<N1>::SEG3 - 1) / (64 / LineSeg<N1>::SEG3);
-  const int nbuv = guv < 65536 ? guv : 65536, nb3 = g3 < 65536 ? g3 : 65536;
-  const size_t luv = lds_uv<N1>(a.NeZ), l3 = lds_3<N1>(a.NeZ);
-  if (l3 > 64 * 1024 || luv > 64 * 1024) {
-    set_error("HEVI: too many elements in the vertical for the line solve's LDS (NeZ)");
+  double* const partial = w->partial;
+  double* const partial_h = w->partial_h;
+  if (!column_fits<N1>(a.NeZ)) {
+    set_error("HEVI: too many elements in the vertical for the line solve (NeZ)");
     return FEDG_ERR_UNSUPPORTED;
   }
+  // wavefronts of the line solves: as many as the scratch holds, walking the
+  // groups of lines from their own slot of it
+  constexpr int WPB = LineSeg<N1>::WPB;
+  const long ngroup = ((long)m.Ne2D * N1 * N1 + LineSeg<N1>::LPW - 1) / LineSeg<N1>::LPW;
+  const size_t list = line_list_doubles(ngroup);
+  const long nwave =
+      w->lines_n <= list ? 0
+                         : std::min((ngroup + WPB - 1) / WPB * WPB,
+                                    (long)((w->lines_n - list) / line_scratch_per_wave(N1, a.NeZ)) / WPB * WPB);
+  if (nwave < WPB || !w->lines) {
+    set_error("HEVI: the line solve's scratch holds no column of this mesh");
+    return FEDG_ERR_UNSUPPORTED;
+  }
+  const dim3 gline((unsigned)(nwave / WPB)), bline(64 * WPB);
+  // usually nothing is flagged: no more workgroups than are resident
+  const dim3 gflag((unsigned)std::min(nwave / WPB, (long)4 * ctx->ncu));
+  a.flagged = reinterpret_cast<int*>(w->lines);
+  a.lines = w->lines + list;
   const long n = (long)m.Np * m.Ne;
   // r0_ext > 0: the residual norm at q^n, the reference of the tolerance when
   // the iteration starts from a predicted iterate (which may already meet it)
@@ -1001,7 +1254,7 @@ int run_newton(fedg_ctx* ctx, HeviArgs& a, int max_it, double rtol, double* resi
       FEDG_HIP_CHECK(hipStreamSynchronize(ctx->stream));
       for (int b = 0; b < 256; ++b) r2 += partial_h[b];
     }
-    hipLaunchKernelGGL(hevi_solve_uv_kernel<N1>, dim3(nbuv), dim3(64), luv, ctx->stream, a);
+    hipLaunchKernelGGL(hevi_solve_uv_kernel<N1>, gline, bline, 0, ctx->stream, a);
     FEDG_HIP_CHECK(hipGetLastError());
     a.pin[VU] = a.pv[VU];
     a.pin[VV] = a.pv[VV];
@@ -1020,7 +1273,13 @@ int run_newton(fedg_ctx* ctx, HeviArgs& a, int max_it, double rtol, double* resi
       if (rtol > 0.0 && it > 0 && r > 0.5 * r_prev) break;
       r_prev = r;
     }
-    hipLaunchKernelGGL(hevi_solve3_kernel<N1>, dim3(nb3), dim3(64), l3, ctx->stream, a);
+    if constexpr (N1 <= 4) {
+      hipLaunchKernelGGL((hevi_solve3_kernel<N1, SOLVE_ALL>), gline, bline, 0, ctx->stream, a);
+    } else {
+      hipLaunchKernelGGL((hevi_solve3_kernel<N1, SOLVE_DIAGONAL>), gline, bline, 0, ctx->stream, a);
+      FEDG_HIP_CHECK(hipGetLastError());
+      hipLaunchKernelGGL((hevi_solve3_kernel<N1, SOLVE_FLAGGED>), gflag, bline, 0, ctx->stream, a);
+    }
     FEDG_HIP_CHECK(hipGetLastError());
     a.pin[VD] = a.pv[VD];
     a.pin[VW] = a.pv[VW];
@@ -1201,7 +1460,7 @@ int hevi_cal_vi(fedg_ctx* ctx, HeviWork* w, double* const tend[5], const double*
         const int rc = predict_iterate<N1>(ctx, w, a, guess, &r0);
         if (rc != FEDG_OK) return rc;
       }
-      const int rc = run_newton<N1>(ctx, a, max_it, rtol, resid, w->partial, w->partial_h, it_done, r0);
+      const int rc = run_newton<N1>(ctx, a, w, max_it, rtol, resid, it_done, r0);
       if (rc != FEDG_OK) return rc;
       const int bs = 256;
       if (store) {
@@ -1282,10 +1541,19 @@ constexpr size_t kScratchDoubles = (size_t)8 << 20;  // 64 MiB
 
 static __device__ __align__(256) double scratch[kScratchDoubles];
 
+// The line solves' scratch of the same calls, apart from it so that the
+// meshes the workspace takes do not change: 32 MiB hold the level solutions
+// of 682 wavefronts at p = 7 and NeZ = 8, and of at least 147 for every
+// column accepted (the wavefronts in flight walk the lines).
+constexpr size_t kLineScratchDoubles = (size_t)4 << 20;
+
+static __device__ __align__(256) double line_scratch[kLineScratchDoubles];
+
 namespace {
 constexpr int kScratchDevices = 64;
 std::mutex scratch_mu;
-double* scratch_dev[kScratchDevices];  // address of `scratch` on each device, set once
+double* scratch_dev[kScratchDevices];       // address of `scratch` on each device, set once
+double* line_scratch_dev[kScratchDevices];  // and of `line_scratch`
 
 // a part of the workspace rounded up to 32 doubles (256 B alignment)
 size_t part(size_t n) { return (n + 31) & ~(size_t)31; }
@@ -1306,12 +1574,14 @@ int noalloc_scratch_setup(int device) {
   }
   std::lock_guard<std::mutex> lock(scratch_mu);
   if (scratch_dev[device]) return FEDG_OK;
-  void* ptr = nullptr;
-  const hipError_t e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
-  if (e != hipSuccess || ptr == nullptr) {
+  void *ptr = nullptr, *lptr = nullptr;
+  hipError_t e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
+  if (e == hipSuccess) e = hipGetSymbolAddress(&lptr, HIP_SYMBOL(line_scratch));
+  if (e != hipSuccess || ptr == nullptr || lptr == nullptr) {
     set_error(std::string("hipGetSymbolAddress of the no-allocation workspace: ") + hipGetErrorString(e));
     return FEDG_ERR_HIP;
   }
+  line_scratch_dev[device] = static_cast<double*>(lptr);
   scratch_dev[device] = static_cast<double*>(ptr);
   return FEDG_OK;
 }
@@ -1364,6 +1634,8 @@ extern "C" int fedg_hevi_cal_vi_noalloc(fedg_ctx* ctx, double* DENS_dt, double* 
   w.coef = p;
   p += part(3 * n);
   w.partial = p;
+  w.lines = line_scratch_dev[ctx->device];
+  w.lines_n = kLineScratchDoubles;
   double* tend[5] = {DENS_dt, RHOT_dt, MOMZ_dt, MOMX_dt, MOMY_dt};
   const double* q[5] = {DDENS_, DRHOT_, MOMZ_, MOMX_, MOMY_};
   const double* q0[5] = {DDENS0_, DRHOT0_, MOMZ0_, MOMX0_, MOMY0_};
