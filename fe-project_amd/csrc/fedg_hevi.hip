@@ -422,16 +422,16 @@ __device__ __forceinline__ bool lu_solve_cols(double (&A)[NS][NS * N], double (&
         off |= here;
         asm volatile("" : "+s"(off));  // compared now: the column's old entries are not kept for later
       } else if (here) {
-        int p = k;
+        // the first largest entry of a column with a larger one (NaN entries
+        // are passed over, a NaN on the diagonal stays, as in the reference's
+        // running comparison)
         double big = fabs(A[sk][k]);
 #pragma unroll
-        for (int i = k + 1; i < n; ++i) {
-          const double t = fabs(A[sk][i]);
-          if (t > big) {
-            big = t;
-            p = i;
-          }
-        }
+        for (int i = k + 1; i < n; ++i) big = __builtin_fmax(big, fabs(A[sk][i]));
+        int p = k;
+#pragma unroll
+        for (int i = n - 1; i > k; --i) p = fabs(A[sk][i]) == big ? i : p;
+        p = larger ? p : k;
         p = bcast_i<SEG, ck>(p);
 #pragma unroll
         for (int i = k + 1; i < n; ++i) {
