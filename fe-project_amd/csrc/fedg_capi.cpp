@@ -99,7 +99,7 @@ struct fedg_heve {
 namespace {
 
 // Horizontally homogeneous base state (every element of a level holds the
-// same values, bit for bit): the p = 7 flat-box kernels read DENS_hyd,
+// same values, bit for bit): the flat-box stage kernels read DENS_hyd,
 // PRES_hyd, THERM_hyd, DPhydDx, DPhydDy (host arrays f) from per-level
 // (5, NeZ, Np) tables, which stay in L2, instead of five full fields.
 // *out stays null when the base state varies horizontally.
@@ -1579,8 +1579,8 @@ int fedg_heve_create(fedg_ctx* ctx, const char* scheme, double dt, const double*
       return FEDG_ERR_HIP;
     }
   }
-  // horizontally homogeneous base state: per-level tables for the flat p = 7 stage
-  if (st->flat && m.n1 == 8) {
+  // horizontally homogeneous base state: per-level tables for the flat-box stages
+  if (st->flat) {
     const double* f[5] = {DENS_hyd, PRES_hyd, THERM_hyd, DPhydDx, DPhydDy};
     rc = level_tables(m, f, &st->lvl);
     if (rc != FEDG_OK) {

@@ -96,7 +96,7 @@ struct TendIn {
   const double* Rtot;        // fused: per node or null (dry constants)
   const double* CVtot;
   const double* CPtot;
-  // fused p = 7 flat stage: DENS_hyd, PRES_hyd, THERM_hyd, DPhydDx, DPhydDy as
+  // fused flat-box stage: DENS_hyd, PRES_hyd, THERM_hyd, DPhydDx, DPhydDy as
   // (5, NeZ, Np) tables by element level when every element of a level holds
   // the same values (horizontally homogeneous base state), else null
   const double* lvl;

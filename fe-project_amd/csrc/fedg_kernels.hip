@@ -7,11 +7,10 @@
 //   1. loads the stage state and base state of its nodes (coalesced, 4 KB per
 //      field per element at p=7),
 //   2. evaluates the Rusanov flux at its NfpTot face nodes (one thread per
-//      face node, exterior values gathered from the neighbour element),
+//      face node, both sides loaded, the exterior one from the neighbour),
 //   3. forms the 15 pointwise fluxes and applies the 1D derivative matrix along
-//      x, y and z through LDS (one variable at a time, double-buffered), adds
-//      the lift of the face flux and the buoyancy / Coriolis / hydrostatic
-//      terms,
+//      x, y and z through LDS, adds the lift of the face flux and the buoyancy
+//      / Coriolis / hydrostatic terms,
 //   4. either writes the five tendencies (drop-in cal_tend) or applies the RK
 //      stage update in place of the reference's separate streaming pass
 //      (fused stepper).
@@ -39,58 +38,128 @@ namespace {
 // overlap the interior work.
 enum { MODE_DROPIN = 0, MODE_FUSED_GENERAL = 1, MODE_FUSED_FLAT = 2, MODE_DROPIN_HEVI = 3, MODE_DROPIN_CCO = 4 };
 
-// Own-node values staged in LDS for the face phase: DDENS, DRHOT, MOMZ, MOMX,
-// MOMY (VID order), then DENS_hyd, PRES_hyd, THERM_hyd, DPRES.
-enum { S_DH = 5, S_PH = 6, S_TH = 7, S_DP = 8, S_N = 9 };
-
-template <int N1, int EPB, int MODE>
-__global__ void __launch_bounds__(EPB * N1 * N1 * N1, 2)
+// Element kernel of every order and mode: EPB elements per workgroup, one
+// thread per node.  FM (drop-in modes; MODE_FUSED_FLAT always): the flat-terrain
+// uniform box the context detected, whose metric arrays hold Gsqrt = GsqrtH =
+// 1, GI3 = 0, axis-aligned unit normals and constant Escale and Fscale: those
+// values are taken as constants, every operation kept.
+//  - Both sides of a face node are loaded straight from memory (the interior
+//    side's lines are the ones the element's own threads load), and the face
+//    flux needs no barrier; only the fluxes, the face jumps and DDENS go
+//    through LDS.
+//  - NB flux buffers: all five variables before one barrier at p = 3..5, two
+//    variables per barrier in four buffers elsewhere (as in heve7_body), where
+//    five would leave fewer workgroups per CU.
+//  - At most 128 VGPRs: four wavefronts per SIMD (the layout that staged the
+//    state in LDS and held every variable's RK operands took 140-226 and left
+//    two).
+//  - The base state comes from the per-level tables where it is horizontally
+//    homogeneous (MODE_FUSED_FLAT), and the RK operands are all loaded before
+//    the first barrier.
+// Bound: HBM traffic and the latency of a chain of loads, barriers and LDS
+// round trips, as the p = 7 stage kernel.  Measured against the layout before:
+// RK4 step at p = 5, 41 x 37 x 13 elements 1.64 -> 1.28 ms; p = 7 over terrain,
+// 27 x 19 x 11 1.46 -> 1.00 ms; drop-in right-hand side at p = 7, 40 x 32 x 16
+// 1.19 -> 0.74 ms (of it 1.01 -> 0.56 ms the tendency).
+// PHYS (fused modes): physics tendencies join the stage's tendency; a kernel
+// of its own because their power keeps registers from everything else.
+template <int N1, int EPB, int MODE, bool FM, bool PHYS = false>
+__global__ void __launch_bounds__(EPB* N1* N1* N1) __attribute__((amdgpu_waves_per_eu(PHYS ? 2 : 4)))
 heve_kernel(const DevMesh m, const Consts c, const TendIn in, const RkOut rk) {
   constexpr int Np = N1 * N1 * N1, Nfp = N1 * N1, NfpTot = 6 * Nfp;
   constexpr bool HEVI = MODE == MODE_DROPIN_HEVI;
   constexpr bool CCO = MODE == MODE_DROPIN_CCO;
   constexpr bool DROPIN = MODE == MODE_DROPIN || HEVI || CCO;
-  constexpr bool FLAT = MODE == MODE_FUSED_FLAT;
+  constexpr bool FLAT = MODE == MODE_FUSED_FLAT;  // neighbours formed arithmetically
   constexpr bool FUSED = !DROPIN;
-  // exterior values are loaded before the first barrier when every face node
-  // has its own thread (p >= 5); otherwise inside the face loop
-  constexpr bool PRELOAD = NfpTot <= Np;
-
+  static_assert(!FLAT || FM, "the arithmetic neighbours are those of the flat box");
+  constexpr int NB = N1 >= 4 && N1 <= 6 ? 5 : 4;
   __shared__ double sDt[N1 * N1];
   __shared__ double sI[N1 * N1];
-  __shared__ double sS[EPB][S_N][Np];
-  __shared__ double sF[2][EPB][3][Np];
-  __shared__ double sDF[EPB][5][NfpTot];
+  __shared__ double sRho[EPB][Np];
+  __shared__ double sF[NB][EPB][3][Np];
+  __shared__ double sDF[EPB][5][CCO ? 1 : NfpTot];
+  __shared__ double sPow[FUSED ? 640 : 1];
 
   const int tid = threadIdx.x;
-  const int e = tid / Np;
+  const int e = EPB == 1 ? 0 : tid / Np;
   const int p = tid - e * Np;
-  int blk = blockIdx.x;
-  if constexpr (FLAT) blk = xcd_remap(blk, gridDim.x);
-  const int ke = blk * EPB + e;
-  const bool valid = ke < m.Ne;
+  const int ke = xcd_remap(blockIdx.x, gridDim.x) * EPB + e;
+  const bool valid = EPB == 1 || ke < m.Ne;
   const int i = p % N1, j = (p / N1) % N1, k = p / Nfp;
   const double gamm = c.CPdry / c.CVdry;
-
-  for (int t = tid; t < N1 * N1; t += blockDim.x) {
+  for (int t = tid; t < N1 * N1; t += EPB * Np) {
     sDt[(t % N1) * N1 + t / N1] = m.D1D[t];
     sI[t] = m.Itr[t];
   }
+  if constexpr (FUSED) pow_tables_to(sPow, tid, EPB * Np);
 
-  // ---- exterior side of this thread's face node: index and boundary kind ----
-  const int fp0 = p;
-  const int f0 = fp0 / Nfp, a0 = fp0 - f0 * Nfp;
-  const bool has_face = valid && fp0 < NfpTot;
-  uint32_t iP0 = 0;
-  int bc0 = FEDG_BND_NONE;
-  const int pm0 = face_node<N1>(f0 < 6 ? f0 : 0, a0);
-  auto exterior = [&](int f, int a, int pm, uint32_t& iP, int& bc) {
-    const uint32_t gf = (uint32_t)(f * Nfp + a) + (uint32_t)NfpTot * ke;
+  // base state: full fields, or (MODE_FUSED_FLAT) the per-level tables
+  const bool lvl = FLAT && in.lvl != nullptr;
+  const int nt = m.NeZ * Np;  // entries of a table
+  const double* const DENS_hyd = lvl ? in.lvl : in.DENS_hyd;
+  const double* const PRES_hyd = lvl ? in.lvl + nt : in.PRES_hyd;
+  const double* const THERM_hyd = lvl ? in.lvl + 2 * nt : in.THERM_hyd;
+  const double* const DPhydDx = lvl ? in.lvl + 3 * nt : in.DPhydDx;
+  const double* const DPhydDy = lvl ? in.lvl + 4 * nt : in.DPhydDy;
+  [[maybe_unused]] int ei = 0, ej = 0, ek = 0;
+  if constexpr (FLAT) {
+    ei = ke % m.NeX;
+    ej = (ke / m.NeX) % m.NeY;
+    ek = ke / (m.NeX * m.NeY);
+  }
+
+  // ---- own node: state, base state, pressure, metric ----
+  const uint32_t o = (uint32_t)Np * (valid ? ke : 0) + p;
+  const uint32_t oh = lvl ? (uint32_t)(Np * (valid ? ek : 0) + p) : o;
+  double q[5] = {0, 0, 0, 0, 0};
+  double Dh = 0, Th = 0, DP = 0;
+  double Gs = 1.0, g13 = 0.0, g23 = 0.0, GsH = 1.0;
+  double E11 = m.fE[0], E22 = m.fE[1], E33 = m.fE[2];
+  int ke2d = 0;
+  if (valid) {
+#pragma unroll
+    for (int v = 0; v < 5; ++v) q[v] = ldg(in.q[v], o);
+    Dh = ldg(DENS_hyd, oh);
+    Th = ldg(THERM_hyd, oh);
+    DP = ldg(in.DPRES, o);
+    ke2d = FLAT ? ei + m.NeX * ej : m.EMap3Dto2D[ke];
+    if constexpr (!FM) {
+      Gs = ldg(m.Gsqrt, o);
+      g13 = ldg(m.G13, o);
+      g23 = ldg(m.G23, o);
+      E11 = ldg(m.E11, o);
+      E22 = ldg(m.E22, o);
+      E33 = ldg(m.E33, o);
+      GsH = ldg(m.GsqrtH, (uint32_t)(i + N1 * j) + (uint32_t)Nfp * ke2d);
+    }
+  }
+  sRho[e][p] = q[VD];
+
+  // ---- face phase: Rusanov flux at the element's face nodes ----
+  auto side = [&](uint32_t n, uint32_t h, Side& S) {
+    S.DD = ldg(in.q[VD], n); S.DT = ldg(in.q[VT], n); S.MZ = ldg(in.q[VW], n);
+    S.MX = ldg(in.q[VU], n); S.MY = ldg(in.q[VV], n);
+    S.Dhyd = ldg(DENS_hyd, h); S.Phyd = ldg(PRES_hyd, h); S.Thyd = ldg(THERM_hyd, h);
+    S.DP = ldg(in.DPRES, n);
+    if constexpr (FM) {
+      S.Gsqrt = 1.0; S.G13 = 0.0; S.G23 = 0.0;
+    } else {
+      S.Gsqrt = ldg(m.Gsqrt, n); S.G13 = ldg(m.G13, n); S.G23 = ldg(m.G23, n);
+    }
+  };
+  // both sides of face node fp; returns the boundary kind of the exterior
+  auto load_face = [&](int fp, Side& M, Side& P) -> int {
+    const int f = fp / Nfp, a = fp - f * Nfp;
+    const int pm = face_node<N1>(f, a);
+    const uint32_t gf = (uint32_t)fp + (uint32_t)NfpTot * ke;
+    uint32_t iP, hP;
+    int bc = FEDG_BND_NONE;
+    const uint32_t iM = DROPIN && !FM ? (uint32_t)m.vmapM[gf] : (uint32_t)Np * ke + pm;
+    uint32_t hM = iM;
     if constexpr (DROPIN) {
-      iP = (uint32_t)m.vmapP[gf];
-      bc = FEDG_BND_NONE;
+      iP = hP = (uint32_t)m.vmapP[gf];
     } else if constexpr (FLAT) {
-      const int ei = ke % m.NeX, ej = (ke / m.NeX) % m.NeY, ek = ke / (m.NeX * m.NeY);
       int ni = ei, nj = ej, nk = ek;
       bool closed = false;
       switch (f) {
@@ -101,186 +170,96 @@ heve_kernel(const DevMesh m, const Consts c, const TendIn in, const RkOut rk) {
         case 4: nk -= 1; if (nk < 0) { if (m.periodic[2]) nk = m.NeZ - 1; else closed = true; } break;
         default: nk += 1; if (nk >= m.NeZ) { if (m.periodic[2]) nk = 0; else closed = true; } break;
       }
+      int nodeP = pm;
+      iP = (uint32_t)Np * ke;
       if (closed) {
-        iP = (uint32_t)Np * ke + pm;
+        nk = ek;
         bc = m.bnd_bc[f];
       } else {
         constexpr int opp[6] = {2, 3, 0, 1, 5, 4};
-        iP = (uint32_t)Np * (ni + m.NeX * (nj + m.NeY * nk)) + face_node<N1>(opp[f], a);
-        bc = FEDG_BND_NONE;
+        nodeP = face_node<N1>(opp[f], a);
+        iP = (uint32_t)Np * (ni + m.NeX * (nj + m.NeY * nk));
       }
+      iP += nodeP;
+      hM = lvl ? (uint32_t)(Np * ek + pm) : iM;
+      hP = lvl ? (uint32_t)(Np * nk + nodeP) : iP;
     } else {
-      iP = (uint32_t)m.nbr[gf];
+      iP = hP = (uint32_t)m.nbr[gf];
       bc = m.nbr_bc[gf];
     }
+    side(iM, hM, M);
+    side(iP, hP, P);
+    return bc;
   };
-  struct Ext {
-    double DD, DT, MZ, MX, MY, Dh, Ph, Th, DP, Gs, g13, g23;
-  };
-  auto load_ext = [&](uint32_t iP, Ext& x) {
-    x.DD = ldg(in.q[VD], iP); x.DT = ldg(in.q[VT], iP); x.MZ = ldg(in.q[VW], iP);
-    x.MX = ldg(in.q[VU], iP); x.MY = ldg(in.q[VV], iP);
-    x.Dh = ldg(in.DENS_hyd, iP); x.Ph = ldg(in.PRES_hyd, iP); x.Th = ldg(in.THERM_hyd, iP);
-    x.DP = ldg(in.DPRES, iP);
-    if constexpr (!FLAT) {
-      x.Gs = ldg(m.Gsqrt, iP); x.g13 = ldg(m.G13, iP); x.g23 = ldg(m.G23, iP);
+  auto face_flux = [&](int fp, int bc, const Side& M, Side& P) {
+    const int f = fp / Nfp;
+    double nx, ny, nz, Fs;
+    if constexpr (FM) {
+      nx = (f == 1) ? 1.0 : (f == 3) ? -1.0 : 0.0;
+      ny = (f == 2) ? 1.0 : (f == 0) ? -1.0 : 0.0;
+      nz = (f == 5) ? 1.0 : (f == 4) ? -1.0 : 0.0;
+      Fs = m.fF[f];
     } else {
-      x.Gs = 1.0; x.g13 = 0.0; x.g23 = 0.0;
+      const uint32_t gf = (uint32_t)fp + (uint32_t)NfpTot * ke;
+      nx = ldg(m.nx, gf);
+      ny = ldg(m.ny, gf);
+      nz = ldg(m.nz, gf);
+      Fs = ldg(m.Fscale, gf);
     }
-  };
-  Ext X0;
-  if constexpr (PRELOAD && !CCO) {
-    if (has_face) {
-      exterior(f0, a0, pm0, iP0, bc0);
-      load_ext(iP0, X0);
+    if (bc != FEDG_BND_NONE) {
+      // exterior momentum from the interior node, as applyBC writes it into the halo
+      double GH = 1.0, g11 = 1.0, g12 = 0.0, g22 = 1.0;
+      if constexpr (!FM) {
+        const int pm = face_node<N1>(f, fp - f * Nfp);
+        const uint32_t h = (uint32_t)(pm % Nfp) + (uint32_t)Nfp * m.EMap3Dto2D[ke];
+        GH = ldg(m.GsqrtH, h);
+        g11 = ldg(m.G11, h);
+        g12 = ldg(m.G12, h);
+        g22 = ldg(m.G22, h);
+      }
+      reflect_momentum(bc, M.Gsqrt, GH, g11, g12, g22, M.G13, M.G23, nx, ny, nz, M.MX, M.MY, M.MZ, P.MX, P.MY, P.MZ);
     }
-  }
-
-  // ---- own node: state, base state, pressure ----
-  const uint32_t o = (uint32_t)Np * (valid ? ke : 0) + p;
-  double q[5] = {0, 0, 0, 0, 0};
-  double Dh = 0, Ph = 0, Th = 0, DP = 0;
-  double Gs = 1.0, g13 = 0.0, g23 = 0.0, GsH = 1.0;
-  int ke2d = 0;
-  double cor = 0.0, dpx = 0.0, dpy = 0.0;
-  if (valid) {
+    double df[5];
+    if constexpr (HEVI) rusanov_hevi(M, P, nx, ny, nz, Fs, gamm, df);
+    else rusanov(M, P, nx, ny, nz, Fs, gamm, df);
 #pragma unroll
-    for (int v = 0; v < 5; ++v) q[v] = ldg(in.q[v], o);
-    Dh = ldg(in.DENS_hyd, o);
-    Ph = ldg(in.PRES_hyd, o);
-    Th = ldg(in.THERM_hyd, o);
-    if constexpr (FLAT) {
-      ke2d = ke % (m.NeX * m.NeY);
+    for (int v = 0; v < 5; ++v) sDF[e][v][fp] = df[v];
+  };
+  if (valid && !CCO) {
+    if constexpr (NfpTot > Np && NfpTot <= 2 * Np) {
+      // two face nodes for some threads (p = 2..4): the second's loads issued
+      // with the first's, one latency instead of two
+      Side M, P, M2, P2;
+      const int fp2 = p + Np;
+      int bc2 = FEDG_BND_NONE;
+      const int bc = load_face(p, M, P);
+      if (fp2 < NfpTot) bc2 = load_face(fp2, M2, P2);
+      face_flux(p, bc, M, P);
+      if (fp2 < NfpTot) face_flux(fp2, bc2, M2, P2);
     } else {
-      Gs = ldg(m.Gsqrt, o);
-      g13 = ldg(m.G13, o);
-      g23 = ldg(m.G23, o);
-      ke2d = m.EMap3Dto2D[ke];
-      GsH = ldg(m.GsqrtH, (uint32_t)(i + N1 * j) + (uint32_t)Nfp * ke2d);
+#pragma unroll 1
+      for (int fp = p; fp < NfpTot; fp += Np) {
+        Side M, P;
+        const int bc = load_face(fp, M, P);
+        face_flux(fp, bc, M, P);
+      }
     }
-    cor = ldg(in.CORIOLIS, (uint32_t)(i + N1 * j) + (uint32_t)Nfp * ke2d);
-    dpx = ldg(in.DPhydDx, o);
-    dpy = ldg(in.DPhydDy, o);
-    DP = ldg(in.DPRES, o);
   }
+  __builtin_amdgcn_sched_barrier(0);
+
+  // ---- volume phase ----
+  const double RDENS = 1.0 / (q[VD] + Dh);
+  const double GsqrtV = Gs / GsH;
+  const double RGsqrtV = 1.0 / GsqrtV;
+  const double RGsqrt = 1.0 / Gs;
   double L[6] = {0, 0, 0, 0, 0, 0};
   if constexpr (!CCO) {
 #pragma unroll
     for (int f = 0; f < 6; ++f) L[f] = ldg(m.Lift, (uint32_t)(p + f * Np));
   }
-#pragma unroll
-  for (int v = 0; v < 5; ++v) sS[e][v][p] = q[v];
-  sS[e][S_DH][p] = Dh;
-  sS[e][S_PH][p] = Ph;
-  sS[e][S_TH][p] = Th;
-  sS[e][S_DP][p] = DP;
-  __syncthreads();
 
-  // ---- face phase: Rusanov flux at the element's face nodes ----
-  if (valid && !CCO) {
-    for (int fp = p; fp < NfpTot; fp += Np) {
-      const int f = fp / Nfp, a = fp - f * Nfp;
-      const int pm = PRELOAD ? pm0 : face_node<N1>(f, a);
-      const uint32_t gf = (uint32_t)fp + (uint32_t)NfpTot * ke;
-      uint32_t iP;
-      int bc;
-      Ext X;
-      if constexpr (PRELOAD) {
-        iP = iP0;
-        bc = bc0;
-        X = X0;
-      } else {
-        exterior(f, a, pm, iP, bc);
-        load_ext(iP, X);
-      }
-      const uint32_t iM = DROPIN ? (uint32_t)m.vmapM[gf] : (uint32_t)Np * ke + pm;
-      const int pmM = DROPIN ? (int)(iM - (uint32_t)Np * ke) : pm;
-      Side M, P;
-      double nx, ny, nz, Fs;
-      if constexpr (FLAT) {
-        nx = (f == 1) ? 1.0 : (f == 3) ? -1.0 : 0.0;
-        ny = (f == 2) ? 1.0 : (f == 0) ? -1.0 : 0.0;
-        nz = (f == 5) ? 1.0 : (f == 4) ? -1.0 : 0.0;
-        Fs = m.fF[f];
-        M.Gsqrt = 1.0; M.G13 = 0.0; M.G23 = 0.0;
-      } else {
-        nx = ldg(m.nx, gf);
-        ny = ldg(m.ny, gf);
-        nz = ldg(m.nz, gf);
-        Fs = ldg(m.Fscale, gf);
-        M.Gsqrt = ldg(m.Gsqrt, iM); M.G13 = ldg(m.G13, iM); M.G23 = ldg(m.G23, iM);
-      }
-      M.DD = sS[e][VD][pmM]; M.DT = sS[e][VT][pmM]; M.MZ = sS[e][VW][pmM];
-      M.MX = sS[e][VU][pmM]; M.MY = sS[e][VV][pmM];
-      M.Dhyd = sS[e][S_DH][pmM]; M.Phyd = sS[e][S_PH][pmM]; M.Thyd = sS[e][S_TH][pmM];
-      M.DP = sS[e][S_DP][pmM];
-      P.Gsqrt = X.Gs; P.G13 = X.g13; P.G23 = X.g23;
-      P.DD = X.DD; P.DT = X.DT; P.MZ = X.MZ; P.MX = X.MX; P.MY = X.MY;
-      P.Dhyd = X.Dh; P.Phyd = X.Ph; P.Thyd = X.Th;
-      P.DP = X.DP;
-      if (bc != FEDG_BND_NONE) {
-        // exterior momentum from the interior node, as applyBC writes it into the halo
-        double GH = 1.0, g11 = 1.0, g12 = 0.0, g22 = 1.0;
-        if constexpr (!FLAT) {
-          const uint32_t h = (uint32_t)(pm % Nfp) + (uint32_t)Nfp * m.EMap3Dto2D[ke];
-          GH = ldg(m.GsqrtH, h);
-          g11 = ldg(m.G11, h);
-          g12 = ldg(m.G12, h);
-          g22 = ldg(m.G22, h);
-        }
-        reflect_momentum(bc, M.Gsqrt, GH, g11, g12, g22, M.G13, M.G23, nx, ny, nz, M.MX, M.MY, M.MZ, P.MX, P.MY,
-                         P.MZ);
-      }
-      double df[5];
-      if constexpr (HEVI) rusanov_hevi(M, P, nx, ny, nz, Fs, gamm, df);
-      else rusanov(M, P, nx, ny, nz, Fs, gamm, df);
-#pragma unroll
-      for (int v = 0; v < 5; ++v) sDF[e][v][fp] = df[v];
-    }
-  }
-
-  // ---- volume phase ----
-  // RK operands, loaded now so their latency overlaps the contractions
-  double rkA[5] = {0, 0, 0, 0, 0}, rkB[5] = {0, 0, 0, 0, 0};
-  if constexpr (FUSED) {
-    if (valid) {
-      if (rk.mode == 1) {
-#pragma unroll
-        for (int v = 0; v < 5; ++v) {
-          rkA[v] = ldg(rk.var0[v], o);
-          rkB[v] = ldg(rk.varTmp[v], o);
-        }
-      } else if (rk.mode == 2) {
-#pragma unroll
-        for (int v = 0; v < 5; ++v) rkB[v] = ldg(rk.varTmp[v], o);
-      }
-    }
-  }
-  const double RDENS = 1.0 / (q[VD] + Dh);
-  const double GsqrtV = Gs / GsH;
-  const double RGsqrtV = 1.0 / GsqrtV;
-  const double RGsqrt = 1.0 / Gs;
-  double E11, E22, E33;
-  if constexpr (FLAT) {
-    E11 = m.fE[0];
-    E22 = m.fE[1];
-    E33 = m.fE[2];
-  } else {
-    E11 = valid ? ldg(m.E11, o) : 0.0;
-    E22 = valid ? ldg(m.E22, o) : 0.0;
-    E33 = valid ? ldg(m.E33, o) : 0.0;
-  }
-  // VFilterPM1 of DDENS (ELM/..._tensorprod3D.F90:2828-2839)
-  double drho = sS[e][VD][i + N1 * j] * sI[N1 * k];
-#pragma unroll
-  for (int l = 1; l < N1; ++l) drho = drho + sS[e][VD][i + N1 * (j + N1 * l)] * sI[l + N1 * k];
-
-  // One variable at a time: pointwise flux (FDS/..._rhot_heve.F90:376-418),
-  // Div_var5 (ELM/..._tensorprod3D.F90:2760-2783: Dx Fx, Dy Fy, Dz Fz and the
-  // lift of del_flux), tendency (:424-483) and its RK update
-  // (CMN/scale_timeint_rk.F90:2232-2350 with one tendency buffer).
-#pragma unroll
-  for (int v = 0; v < 5; ++v) {
+  // pointwise fluxes of a variable (FDS/..._rhot_heve.F90:376-418)
+  auto put_flux = [&](int v) {
     const double m0 = Gs * q[VU];
     const double m1 = Gs * q[VV];
     const double m2 = Gs * (q[VW] * RGsqrtV + g13 * q[VU] + g23 * q[VV]);
@@ -312,28 +291,74 @@ heve_kernel(const DevMesh m, const Consts c, const TendIn in, const RkOut rk) {
       f1 = m1 * v_ + GsqrtDPRES_;
       f2 = m2 * v_ + GsqrtDPRES_ * g23;
     }
-    const int b = v & 1;
+    const int b = v % NB;
     sF[b][e][0][p] = f0;
     sF[b][e][1][p] = f1;
     sF[b][e][2][p] = f2;
-    __syncthreads();
+  };
+
+  // operands of a variable's tendency and RK update, all loaded before the first barrier
+  struct Ops {
+    double rA, rB, s, cor, Ph;
+  };
+  auto load_ops = [&](int v) {
+    Ops op{0.0, 0.0, 0.0, 0.0, 0.0};
+    if (!valid) return op;
+    if constexpr (FUSED) {
+      if (rk.mode == 1) op.rA = ldg_nt(rk.var0[v], o);
+      if (rk.mode == 1 || rk.mode == 2) op.rB = ldg_nt(rk.varTmp[v], o);
+      if (v == VT) op.Ph = ldg(PRES_hyd, oh);
+    }
+    if (v == VU || v == VV) {
+      op.s = ldg(v == VU ? DPhydDx : DPhydDy, oh);
+      op.cor = ldg(in.CORIOLIS, (uint32_t)(i + N1 * j) + (uint32_t)Nfp * ke2d);
+    }
+    return op;
+  };
+  Ops ops[5];
+#pragma unroll
+  for (int v = 0; v < 5; ++v) ops[v] = load_ops(v);
+  double drho = 0.0;
+  // the sum is formed here: without this the compiler forms it where it is
+  // used and keeps (spills) its operands until then
+  auto formed = [&](double& x) {
+    if constexpr (N1 >= 5) asm volatile("" : "+v"(x));
+  };
+  // Div_var5 of a variable (ELM/..._tensorprod3D.F90:2760-2783: Dx Fx, Dy Fy,
+  // Dz Fz and the lift of del_flux), tendency (FDS/..._rhot_heve.F90:424-483)
+  // and its RK update (CMN/scale_timeint_rk.F90:2232-2350 with one tendency
+  // buffer)
+  auto update = [&](int v) {
+    const Ops cur = ops[v];
+    if (v == 0) {
+      // VFilterPM1 of DDENS (ELM/..._tensorprod3D.F90:2828-2839)
+      drho = sRho[e][i + N1 * j] * sI[N1 * k];
+#pragma unroll
+      for (int l = 1; l < N1; ++l) drho = drho + sRho[e][i + N1 * (j + N1 * l)] * sI[l + N1 * k];
+      formed(drho);
+    }
+    const int b = v % NB;
     const double* Fx = sF[b][e][0];
     const double* Fy = sF[b][e][1];
     const double* Fz = sF[b][e][2];
-    // one direction at a time, so that only one line of operands is live
-    // (sDt holds D1D transposed: row i of D1D is sDt[N1*i .. N1*i+N1-1])
-    double dx = sDt[N1 * i] * Fx[N1 * (j + N1 * k)];
+    // sDt holds D1D transposed: row i of D1D is D[N1*i .. N1*i+N1-1].  Read
+    // again for every variable (an offset the compiler cannot see through):
+    // three rows kept in registers would be 6 N1 of them.
+    int zero = 0;
+    asm volatile("" : "+v"(zero));
+    const double* D = sDt + zero;
+    double dx = D[N1 * i] * Fx[N1 * (j + N1 * k)];
 #pragma unroll
-    for (int l = 1; l < N1; ++l) dx = dx + sDt[l + N1 * i] * Fx[l + N1 * (j + N1 * k)];
-    __builtin_amdgcn_sched_barrier(0);
-    double dy = Fy[i + N1 * (N1 * k)] * sDt[N1 * j];
+    for (int l = 1; l < N1; ++l) dx = dx + D[l + N1 * i] * Fx[l + N1 * (j + N1 * k)];
+    formed(dx);
+    double dy = Fy[i + N1 * (N1 * k)] * D[N1 * j];
 #pragma unroll
-    for (int l = 1; l < N1; ++l) dy = dy + Fy[i + N1 * (l + N1 * k)] * sDt[l + N1 * j];
-    __builtin_amdgcn_sched_barrier(0);
-    double dz = Fz[i + N1 * j] * sDt[N1 * k];
+    for (int l = 1; l < N1; ++l) dy = dy + Fy[i + N1 * (l + N1 * k)] * D[l + N1 * j];
+    formed(dy);
+    double dz = Fz[i + N1 * j] * D[N1 * k];
 #pragma unroll
-    for (int l = 1; l < N1; ++l) dz = dz + Fz[i + N1 * (j + N1 * l)] * sDt[l + N1 * k];
-    __builtin_amdgcn_sched_barrier(0);
+    for (int l = 1; l < N1; ++l) dz = dz + Fz[i + N1 * (j + N1 * l)] * D[l + N1 * k];
+    formed(dz);
     const double* dfv = sDF[e][v];
     double X;
     if constexpr (CCO) {
@@ -352,69 +377,86 @@ heve_kernel(const DevMesh m, const Consts c, const TendIn in, const RkOut rk) {
     } else if (v == VW) {
       T = HEVI ? -X * RGsqrt : -X * RGsqrt - c.GRAV * drho;
     } else if (v == VU) {
-      T = -dpx + cor * q[VV];
+      T = -cur.s + cur.cor * q[VV];
       T = T - X * RGsqrt;
     } else {
-      T = -dpy - cor * q[VU];
+      T = -cur.s - cur.cor * q[VU];
       T = T - X * RGsqrt;
     }
+    if (!valid) return;
     if constexpr (FUSED) {
+      double Rt = c.Rdry, Cv = c.CVdry, Cp = c.CPdry;
+      if (v == VT && in.Rtot != nullptr) {
+        Rt = ldg(in.Rtot, o);
+        Cv = ldg(in.CVtot, o);
+        Cp = ldg(in.CPtot, o);
+      }
       // add_phy_tend (FDS/scale_atm_dyn_dgm_driver_nonhydro3d.F90:1098-1178):
       // the physics tendencies join the stage's tendency before the update
-      if (valid && in.tp[0] != nullptr) {
-        if (v == VT) {
-          double Rt = c.Rdry, Cv = c.CVdry, Cp = c.CPdry;
-          if (in.Rtot != nullptr) {
-            Rt = ldg(in.Rtot, o);
-            Cv = ldg(in.CVtot, o);
-            Cp = ldg(in.CPtot, o);
-          }
+      if constexpr (PHYS) {
+        if (v == VT)
           T = phys_add_rhot(T, ldg(in.tp[VT], o), ldg(in.tp[5], o), pres_of(q[VT], Th, Rt, Cv, Cp, c), Rt, Cp, c);
-        } else {
+        else
           T = T + ldg(in.tp[v], o);
-        }
       }
-    }
-    if (valid) {
-      if constexpr (DROPIN) {
-        stg(rk.out[v], o, T);
-      } else {
-        double qn;
-        switch (rk.mode) {
-          case 0:
-            stg(rk.varTmp[v], o, q[v] + rk.cb * T);
-            qn = q[v] + rk.ca * T;
-            break;
-          case 1:
-            stg(rk.varTmp[v], o, rkB[v] + rk.cb * T);
-            qn = rkA[v] + rk.ca * T;
-            break;
-          case 2:
-            qn = rkB[v] + rk.cb * T;
-            break;
-          default:
-            qn = q[v] + rk.cb * T;
-            break;
-        }
-        stg(rk.out[v], o, qn);
-        if (v == VT) {
-          // pressure perturbation of the new state, read by the next stage
-          // (own node and the neighbours' face nodes) instead of recomputed
-          double Rt = c.Rdry, Cv = c.CVdry, Cp = c.CPdry;
-          if (in.Rtot != nullptr) {
-            Rt = ldg(in.Rtot, o);
-            Cv = ldg(in.CVtot, o);
-            Cp = ldg(in.CPtot, o);
-          }
-          stg(rk.DPout, o, dpres_of(qn, Th, Ph, Rt, Cv, Cp, c));
-        }
+      double qn;
+      switch (rk.mode) {
+        case 0:
+          stg_nt(rk.varTmp[v], o, q[v] + rk.cb * T);
+          qn = q[v] + rk.ca * T;
+          break;
+        case 1:
+          stg_nt(rk.varTmp[v], o, cur.rB + rk.cb * T);
+          qn = cur.rA + rk.ca * T;
+          break;
+        case 2:
+          qn = cur.rB + rk.cb * T;
+          break;
+        default:
+          qn = q[v] + rk.cb * T;
+          break;
       }
+      stg_nt(rk.out[v], o, qn);
+      // pressure perturbation of the new state, read by the next stage (own
+      // node and the neighbours' face nodes) instead of recomputed
+      if (v == VT) stg_nt(rk.DPout, o, dpres_of_tab(qn, Th, cur.Ph, Rt, Cv, Cp, c, sPow));
+    } else {
+      stg_nt(rk.out[v], o, T);
     }
-    // finish this variable before the next one's LDS traffic; otherwise the
-    // scheduler defers the arithmetic and every variable's operands stay live
+  };
+  if constexpr (NB == 5) {
+#pragma unroll
+    for (int v = 0; v < 5; ++v) put_flux(v);
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+      update(v);
+      // one variable's operands at a time, or every variable's stay live
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  } else {
+    // variable 4 reuses buffer 0, whose last reads (variable 0) precede the second barrier
+    put_flux(0);
+    put_flux(1);
+    __syncthreads();
+    update(0);
     __builtin_amdgcn_sched_barrier(0);
+    update(1);
+    put_flux(2);
+    put_flux(3);
+    __syncthreads();
+    update(2);
+    __builtin_amdgcn_sched_barrier(0);
+    update(3);
+    put_flux(4);
+    __syncthreads();
+    update(4);
   }
 }
+
+// own-node values staged in LDS by heve32_kernel: DDENS, DRHOT, MOMZ, MOMX,
+// MOMY (VID order), then DENS_hyd, PRES_hyd, THERM_hyd, DPRES
+enum { S_DH = 5, S_PH = 6, S_TH = 7, S_DP = 8, S_N = 9 };
 
 // ---------------------------------------------------------------------------
 // FP32 perturbation form of the fused HEVE stage (flat-terrain box, dry air).
@@ -496,10 +538,17 @@ __device__ __forceinline__ void rusanov32_hevi(const Side32& M, const Side32& P,
 //    lane-varying;
 //  - the pointwise fluxes of two variables go to LDS between barriers (three
 //    barriers per stage), the contractions, lift, tendency and RK update of
-//    each variable follow, the next variable's RK operands loaded ahead;
+//    each variable follow;
 //  - the RK operands are loaded and the stage's outputs stored with the
 //    non-temporal hint (streamed once), so that the state and DPRES lines the
-//    neighbouring elements gather stay in the caches.
+//    neighbouring elements gather stay in the caches; in FP64 all of them are
+//    in flight before the first barrier.
+// Measured (64 x 64 x 16 elements, RK4 step): every sum formed on the spot
+// (124 -> 94 VGPRs) 7.45 -> 7.33 ms, and the RK operands all ahead instead of
+// one variable ahead 7.13 ms (1.78 ms per stage, 3.5 TB/s of HBM traffic);
+// three workgroups per CU with two flux buffers (80 VGPRs, five barriers)
+// 7.71 ms.  FP32 tendency (32 x 32 x 16): 90 -> 76 VGPRs, so three workgroups
+// per CU, 1.78 -> 1.63 ms.
 template <typename R, bool LVL, bool HEVI = false>
 __device__ __forceinline__ void heve7_body(const DevMesh& m, const Consts& c, const TendIn& in, const RkOut& rk,
                                             const int ke) {
@@ -727,7 +776,14 @@ __device__ __forceinline__ void heve7_body(const DevMesh& m, const Consts& c, co
     }
     return op;
   };
-  Ops nxt = load_ops(0);
+  // operands loaded AHEAD variables before their use: in FP64 all of them
+  // before the first barrier (the registers of two workgroups per CU take
+  // them once every contraction is formed on the spot), in FP32, whose three
+  // workgroups per CU hide the latency, one ahead
+  constexpr int AHEAD = F64 ? 5 : 1;
+  Ops ops[5];
+#pragma unroll
+  for (int v = 0; v < AHEAD; ++v) ops[v] = load_ops(v);
   R drho = R(0);
   auto wr = [&](int v) {
     R f0, f1, f2;
@@ -735,9 +791,12 @@ __device__ __forceinline__ void heve7_body(const DevMesh& m, const Consts& c, co
     const int b = v & 3;
     sF[b][0][p] = f0; sF[b][1][p] = f1; sF[b][2][p] = f2;
   };
+  // the sum is formed here: otherwise the compiler forms it where it is used
+  // and keeps its 16 operands until then
+  auto formed = [](R& x) { asm volatile("" : "+v"(x)); };
   auto cu = [&](int v) {
-    const Ops cur = nxt;
-    if (v < 4) nxt = load_ops(v + 1);
+    const Ops cur = ops[v];
+    if (v + AHEAD < 5) ops[v + AHEAD] = load_ops(v + AHEAD);
     const R s = (R)cur.s, cor = (R)cur.cor;
     const int b = v & 3;
     if (v == 0) {
@@ -747,6 +806,7 @@ __device__ __forceinline__ void heve7_body(const DevMesh& m, const Consts& c, co
       drho = zl[0] * sI[N1 * k];
 #pragma unroll
       for (int l = 1; l < N1; ++l) drho = drho + zl[l] * sI[l + N1 * k];
+      formed(drho);
     }
     const R* Fx = sF[b][0];
     const R* Fy = sF[b][1];
@@ -759,6 +819,7 @@ __device__ __forceinline__ void heve7_body(const DevMesh& m, const Consts& c, co
       dx = Di[0] * Fx[N1 * (j + N1 * k)];
 #pragma unroll
       for (int l = 1; l < N1; ++l) dx = dx + Di[l] * Fx[l + N1 * (j + N1 * k)];
+      formed(dx);
     }
     {
       R Dj[N1];
@@ -767,6 +828,7 @@ __device__ __forceinline__ void heve7_body(const DevMesh& m, const Consts& c, co
       dy = Fy[i + N1 * (N1 * k)] * Dj[0];
 #pragma unroll
       for (int l = 1; l < N1; ++l) dy = dy + Fy[i + N1 * (l + N1 * k)] * Dj[l];
+      formed(dy);
     }
     {
       R zl[N1];
@@ -775,6 +837,7 @@ __device__ __forceinline__ void heve7_body(const DevMesh& m, const Consts& c, co
       dz = zl[0] * Dk[0];
 #pragma unroll
       for (int l = 1; l < N1; ++l) dz = dz + zl[l] * Dk[l];
+      formed(dz);
     }
     const R* dfv = sDF[v];
     const R fz4 = dfv[4 * Nfp + i + N1 * j], fz5 = dfv[5 * Nfp + i + N1 * j];
@@ -1642,15 +1705,32 @@ constexpr int epb_for() {
   return (N1 * N1 * N1 >= 128) ? 1 : (256 / (N1 * N1 * N1));
 }
 
+// elements per workgroup of heve_kernel: two at p = 5, whose 216 nodes fill
+// 3.4 wavefronts alone and 6.75 of 7 in pairs
+template <int N1>
+constexpr int heve_epb() {
+  return N1 == 6 ? 2 : epb_for<N1>();
+}
+
 template <int MODE>
 int launch_heve_mode(fedg_ctx* ctx, const TendIn& in, const RkOut& rk) {
   const DevMesh& m = ctx->m;
   auto go = [&](auto n1c) -> int {
     constexpr int N1 = decltype(n1c)::value;
-    constexpr int EPB = epb_for<N1>();
-    const int nblk = (m.Ne + EPB - 1) / EPB;
-    hipLaunchKernelGGL((heve_kernel<N1, EPB, MODE>), dim3(nblk), dim3(EPB * N1 * N1 * N1), 0, ctx->stream, m,
-                       ctx->c, in, rk);
+    constexpr int EPB = heve_epb<N1>();
+    const dim3 g((m.Ne + EPB - 1) / EPB), b(EPB * N1 * N1 * N1);
+    if constexpr (MODE == MODE_FUSED_FLAT || MODE == MODE_FUSED_GENERAL) {
+      constexpr bool FM = MODE == MODE_FUSED_FLAT;
+      if (in.tp[0] != nullptr)
+        hipLaunchKernelGGL((heve_kernel<N1, EPB, MODE, FM, true>), g, b, 0, ctx->stream, m, ctx->c, in, rk);
+      else
+        hipLaunchKernelGGL((heve_kernel<N1, EPB, MODE, FM>), g, b, 0, ctx->stream, m, ctx->c, in, rk);
+    } else {
+      if (m.flat)
+        hipLaunchKernelGGL((heve_kernel<N1, EPB, MODE, true>), g, b, 0, ctx->stream, m, ctx->c, in, rk);
+      else
+        hipLaunchKernelGGL((heve_kernel<N1, EPB, MODE, false>), g, b, 0, ctx->stream, m, ctx->c, in, rk);
+    }
     FEDG_HIP_CHECK(hipGetLastError());
     return FEDG_OK;
   };
