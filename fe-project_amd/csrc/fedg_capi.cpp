@@ -1745,6 +1745,8 @@ static int heve_step(fedg_heve* st, std::vector<hipEvent_t>* evs, size_t* ev_i) 
   const int q0 = st->q0;
   int cur = q0;
   int last_out = q0;
+  // the filter joins the last stage's kernel, except in FP32 and with physics tendencies
+  const bool fuse_filter = st->mfilter && !st->fp32 && !st->tp[0];
   for (int s = 1; s <= t.nstage; ++s) {
     RkOut rk{};
     int outb;
@@ -1765,6 +1767,7 @@ static int heve_step(fedg_heve* st, std::vector<hipEvent_t>* evs, size_t* ev_i) 
     rk.DPout = st->DP[outb];
     rk.cb = t.b_ex[s - 1] * t.dt;
     rk.ca = (s < t.nstage) ? t.dt * t.a_ex[s][s - 1] : 0.0;
+    rk.filter = fuse_filter && s == t.nstage;
     if (st->mflx[0]) {
       // FDS/scale_atm_dyn_dgm_driver_nonhydro3d.F90:899-915: the stage state
       // as the stage's cal_tend sees it (exterior values of the exchange and
@@ -1799,7 +1802,7 @@ static int heve_step(fedg_heve* st, std::vector<hipEvent_t>* evs, size_t* ev_i) 
     last_out = outb;
   }
   st->q0 = last_out;
-  if (st->mfilter) {  // FDS/scale_atm_dyn_dgm_driver_nonhydro3d.F90:940-950
+  if (st->mfilter && !fuse_filter) {  // FDS/scale_atm_dyn_dgm_driver_nonhydro3d.F90:940-950
     double* const* q = st->buf[st->q0];
     TRY(launch_modalfilter(ctx, q[0], q[3], q[4], q[2], q[1], 1));
     const DevMesh& m = ctx->m;

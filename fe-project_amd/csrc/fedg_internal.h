@@ -114,6 +114,7 @@ struct RkOut {
   double ca, cb;             // dt*a(s+1,s), dt*b(s)
   int mode;                  // 0: first stage, 1: middle, 2: last, 3: single-stage scheme,
                              // 4: the tendency itself into out (p = 7 flat-box kernels)
+  int filter;                // FP64 fused, last stage, no physics tendencies: modal filter of the result
 };
 
 int launch_heve_dropin(fedg_ctx* ctx, const TendIn& in, double* const out[5]);

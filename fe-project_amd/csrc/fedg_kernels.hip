@@ -61,10 +61,16 @@ enum { MODE_DROPIN = 0, MODE_FUSED_GENERAL = 1, MODE_FUSED_FLAT = 2, MODE_DROPIN
 // RK4 step at p = 5, 41 x 37 x 13 elements 1.64 -> 1.28 ms; p = 7 over terrain,
 // 27 x 19 x 11 1.46 -> 1.00 ms; drop-in right-hand side at p = 7, 40 x 32 x 16
 // 1.19 -> 0.74 ms (of it 1.01 -> 0.56 ms the tendency).
-// PHYS (fused modes): physics tendencies join the stage's tendency; a kernel
-// of its own because their power keeps registers from everything else.
-template <int N1, int EPB, int MODE, bool FM, bool PHYS = false>
-__global__ void __launch_bounds__(EPB* N1* N1* N1) __attribute__((amdgpu_waves_per_eu(PHYS ? 2 : 4)))
+// KIND (fused modes): STAGE_PHYS, physics tendencies join the stage's tendency
+// (a kernel of its own because their power keeps registers from everything
+// else); STAGE_FILTER, the step's last stage with the modal filter applied to
+// its result, which is element-local (modalfilter_kernel with weighting, then
+// DPRES of the filtered state, operation for operation): two launches and the
+// round trip of the state through memory less (RK4 step at p = 3, 8 x 8 x 4
+// elements: 66.8 -> 60.1 us).
+enum { STAGE_PLAIN = 0, STAGE_PHYS = 1, STAGE_FILTER = 2 };
+template <int N1, int EPB, int MODE, bool FM, int KIND = STAGE_PLAIN>
+__global__ void __launch_bounds__(EPB* N1* N1* N1) __attribute__((amdgpu_waves_per_eu(KIND == STAGE_PHYS ? 2 : 4)))
 heve_kernel(const DevMesh m, const Consts c, const TendIn in, const RkOut rk) {
   constexpr int Np = N1 * N1 * N1, Nfp = N1 * N1, NfpTot = 6 * Nfp;
   constexpr bool HEVI = MODE == MODE_DROPIN_HEVI;
@@ -80,6 +86,8 @@ heve_kernel(const DevMesh m, const Consts c, const TendIn in, const RkOut rk) {
   __shared__ double sF[NB][EPB][3][Np];
   __shared__ double sDF[EPB][5][CCO ? 1 : NfpTot];
   __shared__ double sPow[FUSED ? 640 : 1];
+  constexpr bool PHYS = KIND == STAGE_PHYS, FILTER = KIND == STAGE_FILTER;
+  static_assert(FUSED || KIND == STAGE_PLAIN, "");
 
   const int tid = threadIdx.x;
   const int e = EPB == 1 ? 0 : tid / Np;
@@ -319,6 +327,7 @@ heve_kernel(const DevMesh m, const Consts c, const TendIn in, const RkOut rk) {
 #pragma unroll
   for (int v = 0; v < 5; ++v) ops[v] = load_ops(v);
   double drho = 0.0;
+  [[maybe_unused]] double qf[5];  // STAGE_FILTER: the stage's result
   // the sum is formed here: without this the compiler forms it where it is
   // used and keeps (spills) its operands until then
   auto formed = [&](double& x) {
@@ -416,6 +425,10 @@ heve_kernel(const DevMesh m, const Consts c, const TendIn in, const RkOut rk) {
           qn = q[v] + rk.cb * T;
           break;
       }
+      if constexpr (FILTER) {
+        qf[v] = qn;
+        return;
+      }
       stg_nt(rk.out[v], o, qn);
       // pressure perturbation of the new state, read by the next stage (own
       // node and the neighbours' face nodes) instead of recomputed
@@ -451,6 +464,63 @@ heve_kernel(const DevMesh m, const Consts c, const TendIn in, const RkOut rk) {
     put_flux(4);
     __syncthreads();
     update(4);
+  }
+  if constexpr (FILTER) {
+    // x, y, z passes of the five variables between the two halves of the flux buffers
+    static_assert(NB * 3 >= 10, "");
+    double* A = &sF[0][0][0][0] + (size_t)e * 5 * Np;
+    double* B = A + (size_t)EPB * 5 * Np;
+    const double* Fh = m.MFh;
+    const double* Fv = m.MFv;
+    double h[N1];
+    auto line = [&](const double* row) {
+#pragma unroll
+      for (int l = 0; l < N1; ++l) h[l] = row[N1 * l];
+    };
+    line(Fh + i);
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < 5; ++v) A[v * Np + p] = valid ? Gs * qf[v] : 0.0;
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+      const double* a = A + v * Np + N1 * (j + N1 * k);
+      double x = h[0] * a[0];
+#pragma unroll
+      for (int l = 1; l < N1; ++l) x = x + h[l] * a[l];
+      B[v * Np + p] = x;
+    }
+    line(Fh + j);
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+      const double* b = B + v * Np + i + N1 * N1 * k;
+      double x = b[0] * h[0];
+#pragma unroll
+      for (int l = 1; l < N1; ++l) x = x + b[N1 * l] * h[l];
+      A[v * Np + p] = x;
+    }
+    line(Fv + k);
+    __syncthreads();
+    if (!valid) return;
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+      const double* a = A + v * Np + i + N1 * j;
+      double x = a[0] * h[0];
+#pragma unroll
+      for (int l = 1; l < N1; ++l) x = x + a[Nfp * l] * h[l];
+      x = x * RGsqrt;
+      stg_nt(rk.out[v], o, x);
+      if (v == VT) {
+        double Rt = c.Rdry, Cv = c.CVdry, Cp = c.CPdry;
+        if (in.Rtot != nullptr) {
+          Rt = ldg(in.Rtot, o);
+          Cv = ldg(in.CVtot, o);
+          Cp = ldg(in.CPtot, o);
+        }
+        stg_nt(rk.DPout, o, dpres_of_tab(x, Th, ops[VT].Ph, Rt, Cv, Cp, c, sPow));
+      }
+    }
   }
 }
 
@@ -1722,7 +1792,9 @@ int launch_heve_mode(fedg_ctx* ctx, const TendIn& in, const RkOut& rk) {
     if constexpr (MODE == MODE_FUSED_FLAT || MODE == MODE_FUSED_GENERAL) {
       constexpr bool FM = MODE == MODE_FUSED_FLAT;
       if (in.tp[0] != nullptr)
-        hipLaunchKernelGGL((heve_kernel<N1, EPB, MODE, FM, true>), g, b, 0, ctx->stream, m, ctx->c, in, rk);
+        hipLaunchKernelGGL((heve_kernel<N1, EPB, MODE, FM, STAGE_PHYS>), g, b, 0, ctx->stream, m, ctx->c, in, rk);
+      else if (rk.filter)
+        hipLaunchKernelGGL((heve_kernel<N1, EPB, MODE, FM, STAGE_FILTER>), g, b, 0, ctx->stream, m, ctx->c, in, rk);
       else
         hipLaunchKernelGGL((heve_kernel<N1, EPB, MODE, FM>), g, b, 0, ctx->stream, m, ctx->c, in, rk);
     } else {
@@ -2335,8 +2407,8 @@ int launch_heve_fused32(fedg_ctx* ctx, const TendIn& in, const RkOut& rk) {
 
 int launch_heve_fused(fedg_ctx* ctx, const TendIn& in, const RkOut& rk, int use_flat) {
   const DevMesh& m = ctx->m;
-  // the p = 7 layout carries no physics tendencies: with them, the general layout
-  if (use_flat && m.n1 == 8 && m.lift_tensor && in.tp[0] == nullptr) {
+  // the p = 7 layout carries no physics tendencies and no filter: with them, the general layout
+  if (use_flat && m.n1 == 8 && m.lift_tensor && in.tp[0] == nullptr && !rk.filter) {
     if (in.lvl)
       hipLaunchKernelGGL(heve7_lvl_kernel, dim3(m.Ne), dim3(512), 0, ctx->stream, m, ctx->c, in, rk);
     else
