@@ -712,7 +712,7 @@ int fedg_drhot2pres(fedg_ctx* ctx, double* PRES, double* DPRES, const double* DR
 
 int fedg_halo_exchange(fedg_ctx* ctx, int nfields, double* const* fields) {
   if (!ctx || nfields < 0 || (nfields > 0 && !fields)) return FEDG_ERR_ARG;
-  for (int v = 0; v < nfields; ++v) TRY(launch_halo_exchange(ctx, fields[v]));
+  TRY(launch_halo_exchange(ctx, fields, nfields));
   FEDG_HIP_CHECK(hipStreamSynchronize(ctx->stream));
   return FEDG_OK;
 }
@@ -1231,7 +1231,12 @@ int hevi_work_get(fedg_ctx* ctx, HeviWork** w) {
   al(&h->b3, 3 * n);
   al(&h->buv, 2 * n);
   al(&h->coef, 3 * n);
-  al(&h->partial, 256);
+  if (rc == FEDG_OK &&
+      hipHostMalloc((void**)&h->partial, sizeof(double) * 256 * kHeviPartials, hipHostMallocDefault) != hipSuccess) {
+    set_error("HEVI: host allocation of the residual norms failed");
+    rc = FEDG_ERR_NOMEM;
+  }
+  h->partial_h = h->partial;
   // line-solve scratch: 16 wavefronts per CU (twice what is resident at p = 7,
   // so that the last ones balance), no more than the lines fill
   const size_t lpw = m.n1 <= 4 ? 16 : 8, nline = (size_t)m.Ne2D * m.Nfp;
@@ -1252,11 +1257,12 @@ void hevi_work_free(fedg_ctx* ctx) {
   if (!h) return;
   for (int v = 0; v < 5; ++v)
     if (h->pv[v]) (void)hipFree(h->pv[v]);
-  double* bufs[] = {h->alph, h->b3, h->buv, h->coef, h->lines, h->partial, h->r_plain, h->r_guess, h->flag};
+  double* bufs[] = {h->alph, h->b3, h->buv, h->coef, h->lines, h->r_plain, h->r_guess, h->flag};
   for (double* b : bufs)
     if (b) (void)hipFree(b);
   if (h->X) (void)hipFree(h->X);
   if (h->Y) (void)hipFree(h->Y);
+  if (h->partial) (void)hipHostFree(h->partial);
   delete h;
   ctx->hevi = nullptr;
 }
@@ -2128,12 +2134,10 @@ static int hevi_step(fedg_hevi* st, hipEvent_t* ev) {
     if (!fuse_store)  // StoreImplicit
       TRY(launch_store_implicit(ctx, st->q, Ti, s == 1 ? sto.var0 : nullptr, s == 1 ? sto.varTmp : nullptr,
                                 impl_fac));
-    for (int v = 0; v < 5; ++v) TRY(launch_halo_exchange(ctx, st->q[v]));
     // PRES only for the physics tendencies; dry constants on the verified dry box
-    TRY(launch_drhot2pres(ctx, st->tp[0] ? st->PRES : nullptr, st->DPRES, st->q[1], st->PRES_hyd, st->THERM_hyd,
-                          st->flat7 ? nullptr : st->Rtot, st->flat7 ? nullptr : st->CVtot,
-                          st->flat7 ? nullptr : st->CPtot, n));
-    TRY(launch_halo_exchange(ctx, st->DPRES));
+    TRY(launch_pressure_halo(ctx, st->q, st->tp[0] ? st->PRES : nullptr, st->DPRES, st->PRES_hyd, st->THERM_hyd,
+                             st->flat7 ? nullptr : st->Rtot, st->flat7 ? nullptr : st->CVtot,
+                             st->flat7 ? nullptr : st->CPtot));
     TRY(launch_apply_bc(ctx, st->q[3], st->q[4], st->q[2]));
     TendIn in{};
     for (int v = 0; v < 5; ++v) in.q[v] = st->q[v];

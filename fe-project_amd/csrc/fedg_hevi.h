@@ -4,6 +4,8 @@
 
 namespace fedg {
 
+constexpr int kHeviPartials = 7;
+
 // Device workspace of the implicit solve, allocated once per context.
 struct HeviWork {
   double* pv[5];      // Newton iterate (Np,Ne) per variable
@@ -14,8 +16,8 @@ struct HeviWork {
   double* lines;      // line solves: list of groups to solve with row exchanges, then the level
                       // solutions of the wavefronts in flight
   size_t lines_n;     // doubles in it
-  double* partial;    // 256 partial sums (residual norms)
-  double partial_h[256];
+  double* partial;    // 256 partial sums of each of kHeviPartials vectors (residual norms)
+  double* partial_h;  // where the host reads them: the same memory, or a copy
   // learned initial guess (allocated on first use)
   float* X;           // (chunk, n_in) features
   float* Y;           // (chunk, n_out) predictions

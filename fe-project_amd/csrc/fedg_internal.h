@@ -203,7 +203,11 @@ int launch_dpres(fedg_ctx* ctx, double* DPRES, const double* DRHOT, const double
 int launch_drhot2pres(fedg_ctx* ctx, double* PRES, double* DPRES, const double* DRHOT,
                       const double* PRES_hyd, const double* THERM_hyd, const double* Rtot,
                       const double* CVtot, const double* CPtot, long n);
-int launch_halo_exchange(fedg_ctx* ctx, double* field);
+int launch_halo_exchange(fedg_ctx* ctx, double* const* fields, int nfields);
+// DPRES (and PRES unless null) of the state q with both halos: the exchange of
+// the five variables, DRHOT2PRES and the exchange of DPRES
+int launch_pressure_halo(fedg_ctx* ctx, double* const q[5], double* PRES, double* DPRES, const double* PRES_hyd,
+                         const double* THERM_hyd, const double* Rtot, const double* CVtot, const double* CPtot);
 int launch_apply_bc(fedg_ctx* ctx, double* MOMX, double* MOMY, double* MOMZ);
 int launch_phyd_hgrad(fedg_ctx* ctx, double* DPhydDx, double* DPhydDy, const double* PRES_hyd,
                       const double* PRES_hyd_ref);

@@ -1821,20 +1821,53 @@ int launch_heve_mode(fedg_ctx* ctx, const TendIn& in, const RkOut& rk) {
 }
 
 // ---------------------------------------------------------------------------
-__global__ void drhot2pres_kernel(double* PRES, double* DPRES, const double* DRHOT, const double* PRES_hyd,
-                                  const double* THERM_hyd, const double* Rtot, const double* CVtot,
-                                  const double* CPtot, long n, const Consts c) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
+__device__ __forceinline__ void drhot2pres(double& P, double& DP, const double* DRHOT, const double* PRES_hyd,
+                                           const double* THERM_hyd, const double* Rtot, const double* CVtot,
+                                           const double* CPtot, long t, const Consts& c) {
   const double rP0 = 1.0 / c.PRES00;
   const double RHOT = THERM_hyd[t] + DRHOT[t];
   // null Rtot / CVtot / CPtot: dry air (the caller verified the fields hold
   // the dry constants); null PRES: only DPRES is wanted
   const double Rt = Rtot ? Rtot[t] : c.Rdry;
   const double CVt = CVtot ? CVtot[t] : c.CVdry, CPt = CPtot ? CPtot[t] : c.CPdry;
-  const double P = c.PRES00 * fedg_pow(Rt * rP0 * RHOT, CPt / CVt);
+  P = c.PRES00 * fedg_pow(Rt * rP0 * RHOT, CPt / CVt);
+  DP = P - PRES_hyd[t];
+}
+
+__global__ void drhot2pres_kernel(double* PRES, double* DPRES, const double* DRHOT, const double* PRES_hyd,
+                                  const double* THERM_hyd, const double* Rtot, const double* CVtot,
+                                  const double* CPtot, long n, const Consts c) {
+  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n) return;
+  double P, DP;
+  drhot2pres(P, DP, DRHOT, PRES_hyd, THERM_hyd, Rtot, CVtot, CPtot, t, c);
   if (PRES) PRES[t] = P;
-  DPRES[t] = P - PRES_hyd[t];
+  DPRES[t] = DP;
+}
+
+struct Fields5 {
+  double* f[5];
+};
+
+// drhot2pres_kernel on the n interior nodes; the threads behind them exchange
+// the halo of the five variables and form DPRES there from the node the
+// exchange copies.  One launch where the parts were seven: launches are what a
+// small mesh's stage consists of.
+__global__ void pressure_halo_kernel(const Fields5 q, double* PRES, double* DPRES, const double* PRES_hyd,
+                                     const double* THERM_hyd, const double* Rtot, const double* CVtot,
+                                     const double* CPtot, const int32_t* src, long n, int nB, const Consts c) {
+  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n + nB) return;
+  const long s = t < n ? t : src[t - n];
+  double P, DP;
+  drhot2pres(P, DP, q.f[VT], PRES_hyd, THERM_hyd, Rtot, CVtot, CPtot, s, c);
+  DPRES[t] = DP;
+  if (t < n) {
+    if (PRES) PRES[t] = P;
+    return;
+  }
+#pragma unroll
+  for (int v = 0; v < 5; ++v) q.f[v][t] = q.f[v][s];
 }
 
 __global__ void dpres_kernel(double* DPRES, const double* DRHOT, const double* PRES_hyd, const double* THERM_hyd,
@@ -1850,9 +1883,14 @@ __global__ void dpres_kernel(double* DPRES, const double* DRHOT, const double* P
   DPRES[t] = dpres_of(DRHOT[t], THERM_hyd[t], PRES_hyd[t], Rt, Cv, Cp, c);
 }
 
-__global__ void halo_kernel(double* f, const int32_t* src, long base, int nB) {
+// up to eight fields, one per blockIdx.y
+struct HaloFields {
+  double* f[8];
+};
+__global__ void halo_kernel(const HaloFields h, const int32_t* src, long base, int nB) {
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= nB) return;
+  double* const f = h.f[blockIdx.y];
   f[base + b] = f[src[b]];
 }
 
@@ -2464,11 +2502,28 @@ int launch_dpres(fedg_ctx* ctx, double* DPRES, const double* DRHOT, const double
   return FEDG_OK;
 }
 
-int launch_halo_exchange(fedg_ctx* ctx, double* field) {
+int launch_halo_exchange(fedg_ctx* ctx, double* const* fields, int nfields) {
   const DevMesh& m = ctx->m;
   if (m.nB <= 0) return FEDG_OK;
-  hipLaunchKernelGGL(halo_kernel, dim3(nblocks(m.nB, 256)), dim3(256), 0, ctx->stream, field, m.halo_src,
-                     (long)m.Np * m.Ne, m.nB);
+  for (int v0 = 0; v0 < nfields; v0 += 8) {
+    HaloFields h{};
+    const int nf = std::min(8, nfields - v0);
+    for (int v = 0; v < nf; ++v) h.f[v] = fields[v0 + v];
+    hipLaunchKernelGGL(halo_kernel, dim3(nblocks(m.nB, 256), nf), dim3(256), 0, ctx->stream, h, m.halo_src,
+                       (long)m.Np * m.Ne, m.nB);
+    FEDG_HIP_CHECK(hipGetLastError());
+  }
+  return FEDG_OK;
+}
+
+int launch_pressure_halo(fedg_ctx* ctx, double* const q[5], double* PRES, double* DPRES, const double* PRES_hyd,
+                         const double* THERM_hyd, const double* Rtot, const double* CVtot, const double* CPtot) {
+  const DevMesh& m = ctx->m;
+  const long n = (long)m.Np * m.Ne;
+  Fields5 f;
+  for (int v = 0; v < 5; ++v) f.f[v] = q[v];
+  hipLaunchKernelGGL(pressure_halo_kernel, dim3(nblocks(n + m.nB, 256)), dim3(256), 0, ctx->stream, f, PRES, DPRES,
+                     PRES_hyd, THERM_hyd, Rtot, CVtot, CPtot, m.halo_src, n, m.nB, ctx->c);
   FEDG_HIP_CHECK(hipGetLastError());
   return FEDG_OK;
 }
@@ -2511,10 +2566,6 @@ int launch_phyd_hgrad(fedg_ctx* ctx, double* DPhydDx, double* DPhydDy, const dou
 // applied from the right) and z pass (MFilter_v1D) of
 // element_operation_kernel_matvec_ModalFilter_P* (ELM/..._tensorprod3D_kernel.F90:1061-1112),
 // each sum over l in order, on Gsqrt-weighted values when weight != 0.
-struct Fields5 {
-  double* f[5];
-};
-
 template <int N1, int EPB>
 __global__ void __launch_bounds__(EPB* N1* N1* N1) modalfilter_kernel(Fields5 F, const double* __restrict__ Gsqrt,
                                                                      const double* __restrict__ MFh,
