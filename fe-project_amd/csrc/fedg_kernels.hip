@@ -38,6 +38,7 @@ namespace {
 // overlap the interior work.
 enum { MODE_DROPIN = 0, MODE_FUSED_GENERAL = 1, MODE_FUSED_FLAT = 2, MODE_DROPIN_HEVI = 3, MODE_DROPIN_CCO = 4 };
 
+
 // Element kernel of every order and mode: EPB elements per workgroup, one
 // thread per node.  FM (drop-in modes; MODE_FUSED_FLAT always): the flat-terrain
 // uniform box the context detected, whose metric arrays hold Gsqrt = GsqrtH =
@@ -1255,6 +1256,47 @@ __global__ void __launch_bounds__(EPB * N1 * N1 * N1) heve_bnd_kernel(const DevM
   }
 }
 
+// Sum of s[0 .. N-1] in order from 0 by one lane.  A chain of N additions: eight
+// values are read (s is 16-byte aligned) while the eight before are added, so
+// that the LDS latency stays off the chain.  Lanes that each sum an array of
+// their own run in parallel; stride sum_stride(N) keeps their reads on
+// different banks.
+constexpr int sum_stride(int N) { return (N + 3) & ~1; }
+template <int N>
+__device__ __forceinline__ double ordered_sum(const double* s) {
+  constexpr int U = 8, NB = N / U;
+  typedef double double2_ __attribute__((ext_vector_type(2)));
+  double q = 0.0;
+  if constexpr (NB > 0) {
+    const double2_* v = reinterpret_cast<const double2_*>(s);
+    double2_ a[U / 2], b[U / 2];
+    auto load = [&](double2_(&x)[U / 2], int blk) {
+      const int n = (blk < NB ? blk : NB - 1) * (U / 2);
+#pragma unroll
+      for (int u = 0; u < U / 2; ++u) x[u] = v[n + u];
+    };
+    auto add = [&](const double2_(&x)[U / 2]) {
+#pragma unroll
+      for (int u = 0; u < U / 2; ++u) {
+        q = q + x[u].x;
+        q = q + x[u].y;
+      }
+    };
+    load(a, 0);
+#pragma unroll 1
+    for (int blk = 0; blk + 2 <= NB; blk += 2) {
+      load(b, blk + 1);
+      add(a);
+      load(a, blk + 2);
+      add(b);
+    }
+    if constexpr (NB % 2) add(a);
+  }
+#pragma unroll
+  for (int n = NB * U; n < N; ++n) q = q + s[n];
+  return q;
+}
+
 // Tracer advection tendency, HEVE (FDS/scale_atm_dyn_dgm_trcadvect3d_heve.F90:149-231
 // with its face flux get_delflux_generalhvc, :554-674): central flux of the
 // mass flux with the density's dissipation coefficients alphDENS_M/P, the
@@ -1283,10 +1325,18 @@ enum { TRC_TEND = 0, TRC_FCT = 1 };
 // node in order by one thread.
 // FLAT: the flat-terrain uniform box the context detected (Gsqrt = GsqrtH = 1,
 // GI3 = 0, axis-aligned unit normals, Escale and Fscale constant per
-// direction and face): the same expressions with those exact constants in
-// place of the loads.
+// direction and face, the box's own face map): the same expressions with those
+// exact constants in place of the loads, and the face nodes formed
+// arithmetically except where the neighbour is the halo.
+// Bound: HBM traffic (the tendency 41 KB per element at p = 7, the coefficient
+// 45) behind a chain of gathers, barriers and ordered sums.  The sums' terms
+// are multiplied by the threads that form them; the tendency's line
+// contractions run beside its face sums, the coefficient's mass sum beside
+// its.  48 x 48 x 16 elements at p = 7: tendency 481 -> 468 us, coefficient 449
+// -> 439 us (3.9 TB/s).
 template <int N1, int EPB, int KIND, bool FLAT>
-__global__ void __launch_bounds__(EPB * N1 * N1 * N1) trcadv_kernel(const DevMesh m, const TrcArgs a) {
+__global__ void __launch_bounds__(EPB * N1 * N1 * N1) __attribute__((amdgpu_waves_per_eu(N1 >= 6 ? 8 : 4)))
+trcadv_kernel(const DevMesh m, const TrcArgs a) {
   constexpr int Np = N1 * N1 * N1, Nfp = N1 * N1, NfpTot = 6 * Nfp;
   constexpr bool TEND = KIND == TRC_TEND;
   constexpr int EF = TEND ? EPB : 1;  // arrays only the tendency uses
@@ -1296,10 +1346,11 @@ __global__ void __launch_bounds__(EPB * N1 * N1 * N1) trcadv_kernel(const DevMes
   __shared__ double sDF[EF][TEND ? NfpTot : 1];  // del_flux
   // numflux, QTRC_M MomFlxM and the two fct_coef of this thread's face nodes
   double rNF[NFT], rQF[NFT], rRP[NFT], rRM[NFT];
-  __shared__ double sJF[EPB][NfpTot];            // J(iM) * Fscale * numflux
-  __shared__ double sOut[EPB][6];                // net outward flux of each face
-  __shared__ double sM[TEND ? 1 : EPB][TEND ? 1 : Np];  // FCT: mass terms of the nodes
-  __shared__ double sC[EPB];                            // FCT: the element's coefficient
+  constexpr int SF = sum_stride(Nfp), SM = TEND ? 2 : sum_stride(Np);
+  __shared__ __align__(16) double sJF[EPB][6 * SF];  // FaceIntMat's terms: weight * (J(iM) * Fscale * numflux)
+  __shared__ double sOut[EPB][6];                    // net outward flux of each face
+  __shared__ __align__(16) double sM[TEND ? 1 : EPB][SM];  // FCT: mass terms of the nodes
+  __shared__ double sC[EPB];                               // FCT: the element's mass
   const int tid = threadIdx.x;
   const int e = tid / Np;
   const int p = tid - e * Np;
@@ -1315,15 +1366,39 @@ __global__ void __launch_bounds__(EPB * N1 * N1 * N1) trcadv_kernel(const DevMes
   }
   if constexpr (TEND)
     for (int t = tid; t < N1 * N1; t += blockDim.x) sDt[(t % N1) * N1 + t / N1] = m.D1D[t];
-  const int ke2d = valid ? m.EMap3Dto2D[ke] : 0;
+  const int ke2d = FLAT || !valid ? 0 : m.EMap3Dto2D[ke];
+  [[maybe_unused]] int ei = 0, ej = 0, ek = 0;
+  if constexpr (FLAT) {
+    ei = ke % m.NeX;
+    ej = (ke / m.NeX) % m.NeY;
+    ek = ke / (m.NeX * m.NeY);
+  }
   if (valid) {
 #pragma unroll
     for (int u = 0; u < NFT; ++u) {
       const int fp = p + u * Np;
       if (fp >= NfpTot) break;
       const uint32_t gf = (uint32_t)fp + (uint32_t)NfpTot * ke;
-      const uint32_t iM = (uint32_t)m.vmapM[gf], iP = (uint32_t)m.vmapP[gf];
       const int f = fp / Nfp, an = fp - f * Nfp;
+      uint32_t iM, iP;
+      if constexpr (FLAT) {
+        constexpr int opp[6] = {2, 3, 0, 1, 5, 4};
+        iM = (uint32_t)Np * ke + face_node<N1>(f, an);
+        int step = 0;  // to the neighbour's element
+        bool out = false;
+        switch (f) {
+          case 0: out = ej == 0; step = -m.NeX; break;
+          case 1: out = ei == m.NeX - 1; step = 1; break;
+          case 2: out = ej == m.NeY - 1; step = m.NeX; break;
+          case 3: out = ei == 0; step = -1; break;
+          case 4: out = ek == 0; step = -m.NeX * m.NeY; break;
+          default: out = ek == m.NeZ - 1; step = m.NeX * m.NeY; break;
+        }
+        iP = out ? (uint32_t)m.vmapP[gf] : (uint32_t)Np * (ke + step) + face_node<N1>(opp[f], an);
+      } else {
+        iM = (uint32_t)m.vmapM[gf];
+        iP = (uint32_t)m.vmapP[gf];
+      }
       const double GsH = FLAT ? 1.0 : ldg(m.GsqrtH, (uint32_t)(face_node<N1>(f, an) % Nfp) + (uint32_t)Nfp * ke2d);
       const double Gsqrt_M = FLAT ? 1.0 : ldg(m.Gsqrt, iM), Gsqrt_P = FLAT ? 1.0 : ldg(m.Gsqrt, iP);
       const double GsqrtV_M = Gsqrt_M / GsH, GsqrtV_P = Gsqrt_P / GsH;
@@ -1345,11 +1420,11 @@ __global__ void __launch_bounds__(EPB * N1 * N1 * N1) trcadv_kernel(const DevMes
         rRP[u] = ldg(a.R, iP);
         rRM[u] = ldg(a.R, iM);
       }
-      sJF[e][fp] = ldg(a.J, iM) * (FLAT ? m.fF[f] : ldg(m.Fscale, gf)) * nf;
+      sJF[e][f * SF + an] = (a.w[an % N1] * a.w[an / N1]) * (ldg(a.J, iM) * (FLAT ? m.fF[f] : ldg(m.Fscale, gf)) * nf);
     }
   }
   // volume flux, formed before the face phase's barrier so that its loads
-  // overlap the face gathers (sF is not read before the third barrier)
+  // overlap the face gathers
   double Gs = 1.0, tpo = 0.0;
   if constexpr (TEND) {
     if (valid) {
@@ -1373,29 +1448,40 @@ __global__ void __launch_bounds__(EPB * N1 * N1 * N1) trcadv_kernel(const DevMes
   }
   __syncthreads();
   // FaceIntMat x (J Fscale numflux): row f sums its face's nodes in order from 0
-  if (valid && p < 6) {
-    double s = 0.0;
-#pragma unroll 8
-    for (int an = 0; an < Nfp; ++an) s = s + (a.w[an % N1] * a.w[an / N1]) * sJF[e][p * Nfp + an];
-    sOut[e][p] = s;
-  }
+  if (valid && p < 6) sOut[e][p] = ordered_sum<Nfp>(sJF[e] + p * SF);
   if constexpr (!TEND) {
+    constexpr int PM = Np > 64 ? 64 : 6;  // another wavefront's lane where there is one
+    if (valid && p == PM) sC[e] = ordered_sum<Np>(sM[e]);
     __syncthreads();
-    if (valid && p == 0) {
-      double net = 0.0;
-      for (int f = 0; f < 6; ++f) net = net + (sOut[e][f] > 0.0 ? sOut[e][f] : 0.0);
-      double q = 0.0;
-#pragma unroll 16
-      for (int n = 0; n < Np; ++n) q = q + sM[e][n];
-      double r = q / (net + 1.0e-10);
-      r = r < 1.0 ? r : 1.0;
-      sC[e] = r > 0.0 ? r : 0.0;
-    }
-    __syncthreads();
-    if (valid) stg(a.dt, o, sC[e]);
+    if (!valid) return;
+    double net = 0.0;
+#pragma unroll
+    for (int f = 0; f < 6; ++f) net = net + (sOut[e][f] > 0.0 ? sOut[e][f] : 0.0);
+    double r = sC[e] / (net + 1.0e-10);
+    r = r < 1.0 ? r : 1.0;
+    stg(a.dt, o, r > 0.0 ? r : 0.0);
     return;
   } else {
+    const double* Fx = sF[e][0];
+    const double* Fy = sF[e][1];
+    const double* Fz = sF[e][2];
+    double dx = sDt[N1 * i] * Fx[N1 * (j + N1 * k)];
+#pragma unroll
+    for (int l = 1; l < N1; ++l) dx = dx + sDt[l + N1 * i] * Fx[l + N1 * (j + N1 * k)];
+    // formed here: moved behind the barrier they would keep (spill) their operands
+    asm volatile("" : "+v"(dx));
+    double dy = Fy[i + N1 * (N1 * k)] * sDt[N1 * j];
+#pragma unroll
+    for (int l = 1; l < N1; ++l) dy = dy + Fy[i + N1 * (l + N1 * k)] * sDt[l + N1 * j];
+    asm volatile("" : "+v"(dy));
+    double dz = Fz[i + N1 * j] * sDt[N1 * k];
+#pragma unroll
+    for (int l = 1; l < N1; ++l) dz = dz + Fz[i + N1 * (j + N1 * l)] * sDt[l + N1 * k];
+    asm volatile("" : "+v"(dz));
     __syncthreads();
+    double L[6];
+#pragma unroll
+    for (int f = 0; f < 6; ++f) L[f] = ldg(m.Lift, (uint32_t)(p + f * Np));
     if (valid) {
 #pragma unroll
       for (int u = 0; u < NFT; ++u) {
@@ -1409,21 +1495,6 @@ __global__ void __launch_bounds__(EPB * N1 * N1 * N1) trcadv_kernel(const DevMes
     }
     __syncthreads();
     if (!valid) return;
-    const double* Fx = sF[e][0];
-    const double* Fy = sF[e][1];
-    const double* Fz = sF[e][2];
-    double dx = sDt[N1 * i] * Fx[N1 * (j + N1 * k)];
-#pragma unroll
-    for (int l = 1; l < N1; ++l) dx = dx + sDt[l + N1 * i] * Fx[l + N1 * (j + N1 * k)];
-    double dy = Fy[i + N1 * (N1 * k)] * sDt[N1 * j];
-#pragma unroll
-    for (int l = 1; l < N1; ++l) dy = dy + Fy[i + N1 * (l + N1 * k)] * sDt[l + N1 * j];
-    double dz = Fz[i + N1 * j] * sDt[N1 * k];
-#pragma unroll
-    for (int l = 1; l < N1; ++l) dz = dz + Fz[i + N1 * (j + N1 * l)] * sDt[l + N1 * k];
-    double L[6];
-#pragma unroll
-    for (int f = 0; f < 6; ++f) L[f] = ldg(m.Lift, (uint32_t)(p + f * Np));
     const double* dfv = sDF[e];
     const double lift = L[0] * dfv[i + N1 * k] + L[1] * dfv[Nfp + j + N1 * k] + L[2] * dfv[2 * Nfp + i + N1 * k] +
                         L[3] * dfv[3 * Nfp + j + N1 * k] + L[4] * dfv[4 * Nfp + i + N1 * j] +
@@ -1438,13 +1509,15 @@ __global__ void __launch_bounds__(EPB * N1 * N1 * N1) trcadv_kernel(const DevMes
 // TMAR, the second step of the limiter (:308-337): negative values cut to
 // zero, then the element's tracer mass restored by one factor,
 // QTRC = Q0 / (Q1 + 1e-32) * max(0, QTRC), the two masses summed node by node
-// in order by one thread.
+// in order, each by one thread.  Bound: HBM traffic and the sums' chain; 48 x 48
+// x 16 elements at p = 7 255 -> 187 us (4.0 TB/s).
 template <int N1, int EPB>
 __global__ void __launch_bounds__(EPB * N1 * N1 * N1)
     tmar_kernel(const DevMesh m, double* Q, const double* Dh, const double* DD, const double* J, TrcW w) {
   constexpr int Np = N1 * N1 * N1;
-  __shared__ double s0[EPB][Np], s1[EPB][Np];
-  __shared__ double sr[EPB];
+  constexpr int S = sum_stride(Np);
+  __shared__ __align__(16) double s[EPB][2][S];
+  __shared__ double sr[EPB][2];
   const int tid = threadIdx.x;
   const int e = tid / Np;
   const int p = tid - e * Np;
@@ -1457,32 +1530,27 @@ __global__ void __launch_bounds__(EPB * N1 * N1 * N1)
     const double dens = ldg(Dh, o) + ldg(DD, o);
     const double q = ldg(Q, o);
     qp = q > 0.0 ? q : 0.0;
-    const double g = ldg(m.Gsqrt, o) * ldg(J, o) * ((w.w[i] * w.w[j]) * w.w[k]) * dens;
-    s0[e][p] = g * q;
-    s1[e][p] = g * qp;
+    const double g = (m.flat ? 1.0 : ldg(m.Gsqrt, o)) * ldg(J, o) * ((w.w[i] * w.w[j]) * w.w[k]) * dens;
+    s[e][0][p] = g * q;
+    s[e][1][p] = g * qp;
   }
   __syncthreads();
-  if (valid && p == 0) {
-    double q0 = 0.0, q1 = 0.0;
-#pragma unroll 16
-    for (int n = 0; n < Np; ++n) {
-      q0 = q0 + s0[e][n];
-      q1 = q1 + s1[e][n];
-    }
-    sr[e] = q0 / (q1 + 1.0e-32);
-  }
+  if (valid && p < 2) sr[e][p] = ordered_sum<Np>(s[e][p]);
   __syncthreads();
-  if (valid) stg(Q, o, sr[e] * qp);
+  if (valid) stg(Q, o, sr[e][0] / (sr[e][1] + 1.0e-32) * qp);
 }
 
 // ATMOS_THERMODYN_specific_heat of the SCALE library (scale_atmos_thermodyn,
 // not part of the reference tree; the published mixing rule): qdry = 1 -
 // sum q_i M_i, Rtot = sum q_i R_i + qdry Rdry, likewise CVtot and CPtot, the
 // sums over the tracers in order.
-__device__ __forceinline__ void specific_heat(const double* q, const TrcThermo& th, const Consts& c, double& R,
+template <int NQ>
+__device__ __forceinline__ void specific_heat(const double (&q)[NQ], const TrcThermo& th, const Consts& c, double& R,
                                               double& CV, double& CP) {
   double qdry = 1.0, r = 0.0, cv = 0.0, cp = 0.0;
-  for (int iq = 0; iq < th.nq; ++iq) {
+#pragma unroll
+  for (int iq = 0; iq < NQ; ++iq) {
+    if (iq >= th.nq) break;
     qdry = qdry - q[iq] * th.Mq[iq];
     r = r + q[iq] * th.Rq[iq];
     cv = cv + q[iq] * th.CVq[iq];
@@ -1502,7 +1570,9 @@ __global__ void __launch_bounds__(256) specific_heat_kernel(const SpecHeat a, co
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n) return;
   double q[kMaxTrc];
-  for (int iq = 0; iq < a.th.nq; ++iq) q[iq] = a.Q[iq][t];
+#pragma unroll
+  for (int iq = 0; iq < kMaxTrc; ++iq)
+    if (iq < a.th.nq) q[iq] = a.Q[iq][t];
   double R, CV, CP;
   specific_heat(q, a.th, c, R, CV, CP);
   a.R[t] = R;
@@ -1578,12 +1648,19 @@ __global__ void __launch_bounds__(256) diagvar_kernel(const DiagVar a, const Con
 // over the nodes in order by one thread, as Fortran's sum over p = 1..Np.
 // The water species are all nq tracers (the reference's loop over
 // 1 + QLA + QIA; its later loop over QA reads only those).
-template <int N1, int EPB>
-__global__ void __launch_bounds__(EPB * N1 * N1 * N1) negfix_kernel(const DevMesh m, const Consts c, const NegFix a) {
+// Bound: the ordered sums' chains, then HBM traffic.  No species' sums depend on
+// another's correction, so all of them are formed at once, a lane each: two
+// chains per element where there were nq + 1.  NQ: room for species; four keep
+// the sums' terms at 33 KB per element of p = 7.  32 x 32 x 16 elements, three
+// species: 895 -> 371 us.
+template <int N1, int EPB, int NQ>
+__global__ void __launch_bounds__(EPB * N1 * N1 * N1) __attribute__((amdgpu_waves_per_eu(NQ == 4 && N1 == 8 ? 8 : 4)))
+negfix_kernel(const DevMesh m, const Consts c, const NegFix a) {
   constexpr int Np = N1 * N1 * N1;
   constexpr double TRC_EPS = 1.0e-128;
-  __shared__ double s0[EPB][Np], s1[EPB][Np];
-  __shared__ double sr[EPB][2];
+  constexpr int S = sum_stride(Np);
+  __shared__ __align__(16) double s[EPB][2 * NQ][S];
+  __shared__ double sr[EPB][2 * NQ];
   const int tid = threadIdx.x;
   const int e = tid / Np;
   const int p = tid - e * Np;
@@ -1594,62 +1671,58 @@ __global__ void __launch_bounds__(EPB * N1 * N1 * N1) negfix_kernel(const DevMes
   const int nq = a.th.nq;
   double DENS = 0.0, DD0 = 0.0, DD = 0.0, IE0 = 0.0, TEMP = 0.0, IE = 0.0, intw = 0.0;
   double Dh = 0.0;
-  double tm1[kMaxTrc];
+  double tm0[NQ], qn[NQ];  // qn: the corrected masses, then the species
   if (valid) {
     Dh = ldg(a.Dh, o);
     DD = ldg(a.DD, o);
     DENS = Dh + DD;
     DD0 = DD;
+#pragma unroll
+    for (int iq = 0; iq < NQ; ++iq)
+      if (iq < nq) tm0[iq] = DENS * ldg(a.Q[iq], o);
     const double CV = ldg(a.CV, o), P = ldg(a.PRES, o), R = ldg(a.R, o);
     IE0 = CV * P / R;
     TEMP = IE0 / (DENS * CV);
     IE = IE0;
-    intw = ldg(m.Gsqrt, o) * ldg(a.J, o) * ((a.w.w[i] * a.w.w[j]) * a.w.w[k]);
-  }
-  auto esum = [&](double v0, double v1, double& r0, double& r1) {
-    s0[e][p] = v0;
-    s1[e][p] = v1;
-    __syncthreads();
-    if (valid && p == 0) {
-      double q0 = 0.0, q1 = 0.0;
-#pragma unroll 16
-      for (int n = 0; n < Np; ++n) {
-        q0 = q0 + s0[e][n];
-        q1 = q1 + s1[e][n];
+    intw = (m.flat ? 1.0 : ldg(m.Gsqrt, o)) * ldg(a.J, o) * ((a.w.w[i] * a.w.w[j]) * a.w.w[k]);
+#pragma unroll
+    for (int iq = 0; iq < NQ; ++iq)
+      if (iq < nq) {
+        qn[iq] = tm0[iq] > TRC_EPS ? tm0[iq] : TRC_EPS;
+        s[e][2 * iq][p] = intw * tm0[iq];
+        s[e][2 * iq + 1][p] = intw * qn[iq];
       }
-      sr[e][0] = q0;
-      sr[e][1] = q1;
-    }
+  }
+  // the element sums of the first n arrays
+  auto sums = [&](int n) {
     __syncthreads();
-    r0 = sr[e][0];
-    r1 = sr[e][1];
+    if (valid)
+      for (int v = p; v < n; v += Np) sr[e][v] = ordered_sum<Np>(s[e][v]);
     __syncthreads();
   };
-  for (int iq = 0; iq < nq; ++iq) {
-    double tm0 = 0.0, t1 = 0.0;
-    if (valid) {
-      tm0 = DENS * ldg(a.Q[iq], o);
-      t1 = tm0 > TRC_EPS ? tm0 : TRC_EPS;
-    }
-    double M0, M1;
-    esum(intw * tm0, intw * t1, M0, M1);
-    if (valid) {
-      t1 = (M0 > 0.0 ? M0 : 0.0) / M1 * t1;
-      DD = DD + (t1 - tm0);
-      IE = IE + (t1 - tm0) * a.th.CVq[iq] * TEMP;
-    }
-    tm1[iq] = t1;
-  }
-  double qn[kMaxTrc];
+  sums(2 * nq);
   if (valid) {
+#pragma unroll
+    for (int iq = 0; iq < NQ; ++iq)
+      if (iq < nq) {
+        const double M0 = sr[e][2 * iq], M1 = sr[e][2 * iq + 1];
+        const double t1 = (M0 > 0.0 ? M0 : 0.0) / M1 * qn[iq];
+        DD = DD + (t1 - tm0[iq]);
+        IE = IE + (t1 - tm0[iq]) * a.th.CVq[iq] * TEMP;
+        qn[iq] = t1;
+      }
     DENS = Dh + DD;
-    for (int iq = 0; iq < nq; ++iq) {
-      qn[iq] = tm1[iq] / DENS;
-      stg(a.Q[iq], o, qn[iq]);
-    }
+#pragma unroll
+    for (int iq = 0; iq < NQ; ++iq)
+      if (iq < nq) {
+        qn[iq] = qn[iq] / DENS;
+        stg(a.Q[iq], o, qn[iq]);
+      }
+    s[e][0][p] = intw * IE0;
+    s[e][1][p] = intw * IE;
   }
-  double E0, E1;
-  esum(intw * IE0, intw * IE, E0, E1);
+  sums(2);
+  const double E0 = sr[e][0], E1 = sr[e][1];
   if (!valid) return;
   IE = E0 / E1 * IE;
   double R, CV, CP;
@@ -2261,8 +2334,9 @@ int launch_negative_fixer(fedg_ctx* ctx, const NegFix& a) {
     constexpr int N1 = decltype(n1c)::value;
     constexpr int EPB = epb_for<N1>();
     const int nblk = (m.Ne + EPB - 1) / EPB;
-    hipLaunchKernelGGL((negfix_kernel<N1, EPB>), dim3(nblk), dim3(EPB * N1 * N1 * N1), 0, ctx->stream, m, ctx->c,
-                       a);
+    const dim3 g(nblk), b(EPB * N1 * N1 * N1);
+    if (a.th.nq <= 4) hipLaunchKernelGGL((negfix_kernel<N1, EPB, 4>), g, b, 0, ctx->stream, m, ctx->c, a);
+    else hipLaunchKernelGGL((negfix_kernel<N1, EPB, kMaxTrc>), g, b, 0, ctx->stream, m, ctx->c, a);
     FEDG_HIP_CHECK(hipGetLastError());
     return FEDG_OK;
   });
