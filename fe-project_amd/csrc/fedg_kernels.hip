@@ -38,6 +38,15 @@ namespace {
 // overlap the interior work.
 enum { MODE_DROPIN = 0, MODE_FUSED_GENERAL = 1, MODE_FUSED_FLAT = 2, MODE_DROPIN_HEVI = 3, MODE_DROPIN_CCO = 4 };
 
+// The node's entry of Lift_mat for face f.  Where the matrix has the
+// tensor-product structure the entry depends on the index along the face's
+// normal alone and comes from the n1 x 6 table: a few lines instead of all 6 Np
+// entries per element (24 KB at p = 7).
+template <int N1>
+__device__ __forceinline__ double lift_entry(const DevMesh& m, int f, int i, int j, int k) {
+  if (m.lift_tensor) return ldg(m.liftT, (uint32_t)((f >= 4 ? k : f == 1 || f == 3 ? i : j) + N1 * f));
+  return ldg(m.Lift, (uint32_t)(i + N1 * (j + N1 * k) + f * (N1 * N1 * N1)));
+}
 
 // Element kernel of every order and mode: EPB elements per workgroup, one
 // thread per node.  FM (drop-in modes; MODE_FUSED_FLAT always): the flat-terrain
@@ -264,7 +273,7 @@ heve_kernel(const DevMesh m, const Consts c, const TendIn in, const RkOut rk) {
   double L[6] = {0, 0, 0, 0, 0, 0};
   if constexpr (!CCO) {
 #pragma unroll
-    for (int f = 0; f < 6; ++f) L[f] = ldg(m.Lift, (uint32_t)(p + f * Np));
+    for (int f = 0; f < 6; ++f) L[f] = lift_entry<N1>(m, f, i, j, k);
   }
 
   // pointwise fluxes of a variable (FDS/..._rhot_heve.F90:376-418)
@@ -1244,7 +1253,7 @@ __global__ void __launch_bounds__(EPB * N1 * N1 * N1) heve_bnd_kernel(const DevM
   const uint32_t o = (uint32_t)Np * ke + p;
   double L[6];
 #pragma unroll
-  for (int f = 0; f < 6; ++f) L[f] = ldg(m.Lift, (uint32_t)(p + f * Np));
+  for (int f = 0; f < 6; ++f) L[f] = lift_entry<N1>(m, f, i, j, k);
   const double RGsqrt = 1.0 / ldg(m.Gsqrt, o);
 #pragma unroll
   for (int v = 0; v < 5; ++v) {
@@ -1481,7 +1490,7 @@ trcadv_kernel(const DevMesh m, const TrcArgs a) {
     __syncthreads();
     double L[6];
 #pragma unroll
-    for (int f = 0; f < 6; ++f) L[f] = ldg(m.Lift, (uint32_t)(p + f * Np));
+    for (int f = 0; f < 6; ++f) L[f] = lift_entry<N1>(m, f, i, j, k);
     if (valid) {
 #pragma unroll
       for (int u = 0; u < NFT; ++u) {
