@@ -55,13 +55,37 @@ struct HeviArgs {
   double* b3;              // (3, Np*Ne): DENS, MOMZ, RHOT rhs
   double* buv;             // (2, Np*Ne)
   double* coef;            // (3, Np*Ne): POT, WT, DPDRHOT
-  double* T[5];            // implicit-operator tendencies (VID order), written when want_T
+  double* T[5];            // implicit-operator tendencies (VID order)
   int* flagged;            // groups of lines whose pivots leave the diagonal: their number, then the groups
   double* lines;           // scratch of the line solves: the level solutions of every wavefront in flight
   double impl_fac;
   int want_b;              // form the rhs (Newton) or only the operator (impl_fac = 0)
   int NeZ;
+  int finish;              // FINISH_*: what the line solves store
+  double* qst[5];          // StoreImplicit: the stage state as written (qs), and its copies
+  double* var0[5];
+  double* varTmp[5];
 };
+// What the solve of DENS, MOMZ and RHOT stores: the iterate; or, in the last
+// iteration of a fixed number, what hevi_tend_store_kernel would form from it.
+// The solve is bound by its arithmetic, so the stores hide behind it; MOMX and
+// MOMY, whose solve is not (143 -> 206 us with them) and whose iterate the others'
+// residual reads, stay with the kernel.  60 x 16 x 8 elements at p = 7, a stage:
+// solve 776 -> 808 us, the kernel behind it 104 -> 42 us; drop-in solve of
+// 240 x 16 x 8 elements 4848 -> 4683 us.
+enum { FINISH_NONE = 0, FINISH_TEND = 1, FINISH_STORE = 2, FINISH_STORE_COPY = 3 };
+
+// a node's value P of the iterate, qs = q* there
+__device__ __forceinline__ void finish_node(const HeviArgs& a, int v, uint32_t o, double P, double qs) {
+  const double T = (P - qs) / a.impl_fac;
+  stg_nt(a.T[v], o, T);
+  if (a.finish == FINISH_TEND) return;
+  if (a.finish == FINISH_STORE_COPY) {
+    stg_nt(a.var0[v], o, qs);
+    stg_nt(a.varTmp[v], o, qs);
+  }
+  stg(a.qst[v], o, qs + a.impl_fac * T);
+}
 
 __device__ __forceinline__ double gsqrtv(const HeviArgs& a, int ke, int p, int N1) {
   const int ke2d = a.m.EMap3Dto2D[ke];
@@ -900,7 +924,7 @@ hevi_solve3_kernel(const HeviArgs a) {
     const int tid = opaque(threadIdx.x), c = tid % SEG, pv = c < N ? c : N - 1;
     const bool lv = g * LPW + (tid & 63) / SEG < nline;
     const int line = line_of(tid), ke2D = line / Nfp, ij = line % Nfp;
-    double y[3] = {0.0, 0.0, 0.0}, x[3][4], p0[3];
+    double y[3] = {0.0, 0.0, 0.0}, x[3][4], p0[3], s[3] = {0.0, 0.0, 0.0};
     auto back = [&](int kz) __attribute__((always_inline)) {  // loads of a level, issued one level ahead
       const double* xk = scr + (size_t)kz * n3 * (4 * LPW);
       const uint32_t o = (uint32_t)(3 * pv * (4 * LPW) + (tid & 63) / SEG * 4);
@@ -912,10 +936,16 @@ hevi_solve3_kernel(const HeviArgs a) {
       p0[0] = ldg(a.pin[VD], q);
       p0[1] = ldg(a.pin[VW], q);
       p0[2] = ldg(a.pin[VT], q);
+      if (a.finish) {
+        s[0] = ldg_nt(a.qs[VD], q);
+        s[1] = ldg_nt(a.qs[VW], q);
+        s[2] = ldg_nt(a.qs[VT], q);
+      }
     };
     back(NeZ - 1);
     for (int kz = NeZ - 1; kz >= 0; --kz) {
       double y0[3], z[3][4], o[3];
+      const double sD = s[0], sW = s[1], sT = s[2];
 #pragma unroll
       for (int v = 0; v < 3; ++v) {
         y0[v] = bcast<SEG, 0>(y[v]);
@@ -931,50 +961,47 @@ hevi_solve3_kernel(const HeviArgs a) {
       }
       if (lv && c < N) {
         const uint32_t q = (uint32_t)(Np * (ke2D + kz * m.Ne2D) + ij + Nfp * pv);
-        stg(a.pv[VD], q, o[0] + y[0]);
-        stg(a.pv[VW], q, o[1] + y[1]);
-        stg(a.pv[VT], q, o[2] + y[2]);
+        if (a.finish) {
+          finish_node(a, VD, q, o[0] + y[0], sD);
+          finish_node(a, VW, q, o[1] + y[1], sW);
+          finish_node(a, VT, q, o[2] + y[2], sT);
+        } else {
+          stg(a.pv[VD], q, o[0] + y[0]);
+          stg(a.pv[VW], q, o[1] + y[1]);
+          stg(a.pv[VT], q, o[2] + y[2]);
+        }
       }
     }
     wave_sync();
   }
 }
 
-// tendency = (iterate - q*) / impl_fac  (..._rhot_hevi.F90:937-947)
-__global__ void hevi_tend_kernel(double* T0, double* T1, double* T2, double* T3, double* T4, const double* p0,
-                                 const double* p1, const double* p2, const double* p3, const double* p4,
-                                 const double* q0, const double* q1, const double* q2, const double* q3,
-                                 const double* q4, double impl_fac, long n) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  T0[t] = (p0[t] - q0[t]) / impl_fac;
-  T1[t] = (p1[t] - q1[t]) / impl_fac;
-  T2[t] = (p2[t] - q2[t]) / impl_fac;
-  T3[t] = (p3[t] - q3[t]) / impl_fac;
-  T4[t] = (p4[t] - q4[t]) / impl_fac;
-}
-
-// the same tendency, then the stepper's StoreImplicit on the node: var0 and
-// varTmp (first stage) take q, and q = q + impl_fac T (streamed: non-temporal
-// loads and stores)
+// tendency = (iterate - q*) / impl_fac (..._rhot_hevi.F90:937-947) of nv
+// variables and, as finish says, the stepper's StoreImplicit on the node: var0
+// and varTmp (first stage) take q, and q = q + impl_fac T (streamed:
+// non-temporal loads and stores).
 struct TendStore {
+  int nv;
   double* T[5];
   const double* p[5];
+  const double* qs[5];
   double* q[5];
   double* var0[5];
   double* varTmp[5];
   double impl_fac;
-  int copy;
+  int finish;
 };
 __global__ void hevi_tend_store_kernel(const TendStore a, long n) {
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n) return;
 #pragma unroll
   for (int v = 0; v < 5; ++v) {
-    const double q = __builtin_nontemporal_load(a.q[v] + t);
+    if (v >= a.nv) break;
+    const double q = __builtin_nontemporal_load(a.qs[v] + t);
     const double T = (__builtin_nontemporal_load(a.p[v] + t) - q) / a.impl_fac;
     __builtin_nontemporal_store(T, a.T[v] + t);
-    if (a.copy) {
+    if (a.finish == FINISH_TEND) continue;
+    if (a.finish == FINISH_STORE_COPY) {
       __builtin_nontemporal_store(q, a.var0[v] + t);
       __builtin_nontemporal_store(q, a.varTmp[v] + t);
     }
@@ -1209,9 +1236,12 @@ bool column_fits(int NeZ) {
   return sizeof(double) * l3 <= 64 * 1024 && sizeof(double) * lu <= 64 * 1024;
 }
 
+// finish: what the solve of DENS, MOMZ and RHOT of the last iteration stores,
+// where that iteration is known beforehand (no tolerance, no residual asked
+// for); FINISH_NONE is left in a.finish where it stored the iterate instead
 template <int N1>
 int run_newton(fedg_ctx* ctx, HeviArgs& a, HeviWork* w, int max_it, double rtol, double* resid, int* it_done,
-               double r0_ext = 0.0) {
+               double r0_ext, int finish) {
   const DevMesh& m = ctx->m;
   double* const partial = w->partial;
   double* const partial_h = w->partial_h;
@@ -1262,11 +1292,12 @@ int run_newton(fedg_ctx* ctx, HeviArgs& a, HeviWork* w, int max_it, double rtol,
   }
   double r_prev = 0.0;
   int it = 0;
+  const bool track = rtol > 0.0 || resid != nullptr;
   for (; it < max_it; ++it) {
+    a.finish = !track && it == max_it - 1 ? finish : FINISH_NONE;
     launch_rhs_uv<N1>(ctx, a);
     FEDG_HIP_CHECK(hipGetLastError());
     a.alph_ready = 1;  // the damping coefficients depend on q0 alone
-    const bool track = rtol > 0.0 || resid != nullptr;
     hipLaunchKernelGGL(hevi_solve_uv_kernel<N1>, gline, bline, 0, ctx->stream, a);
     FEDG_HIP_CHECK(hipGetLastError());
     a.pin[VU] = a.pv[VU];
@@ -1431,7 +1462,7 @@ int hevi_cal_vi(fedg_ctx* ctx, HeviWork* w, double* const tend[5], const double*
                 const double* const var0[5], const double* DENS_hyd, const double* PRES_hyd, const double* Rtot,
                 const double* CVtot, const double* CPtot, double impl_fac, int max_it, double rtol, double* resid,
                 int* it_done, HeviGuess* guess, const HeviStore* store, const double* RHOT_hyd,
-                int alph_ready) {
+                int alph_ready, int keep_iterate) {
   const DevMesh& m = ctx->m;
   if (store && !(fabs(impl_fac) > 0.0)) {
     set_error("hevi_cal_vi: the fused StoreImplicit needs impl_fac != 0");
@@ -1481,31 +1512,35 @@ int hevi_cal_vi(fedg_ctx* ctx, HeviWork* w, double* const tend[5], const double*
         const int rc = predict_iterate<N1>(ctx, w, a, guess, &r0);
         if (rc != FEDG_OK) return rc;
       }
-      const int rc = run_newton<N1>(ctx, a, w, max_it, rtol, resid, it_done, r0);
-      if (rc != FEDG_OK) return rc;
-      const int bs = 256;
-      if (store) {
-        TendStore ts{};
+      const int finish = !store ? FINISH_TEND : store->var0[0] ? FINISH_STORE_COPY : FINISH_STORE;
+      if (store)
         for (int v = 0; v < 5; ++v) {
-          ts.T[v] = tend[v];
-          ts.p[v] = w->pv[v];
-          ts.q[v] = store->q[v];
-          ts.var0[v] = store->var0[v];
-          ts.varTmp[v] = store->varTmp[v];
           if (store->q[v] != q[v]) {
             set_error("hevi_cal_vi: the StoreImplicit state is not the solve's stage state");
             return FEDG_ERR_ARG;
           }
+          a.qst[v] = store->q[v];
+          a.var0[v] = store->var0[v];
+          a.varTmp[v] = store->varTmp[v];
         }
-        ts.copy = store->var0[0] != nullptr;
-        ts.impl_fac = impl_fac;
-        hipLaunchKernelGGL(hevi_tend_store_kernel, dim3((n + bs - 1) / bs), dim3(bs), 0, ctx->stream, ts, n);
-        FEDG_HIP_CHECK(hipGetLastError());
-        return FEDG_OK;
+      const int rc = run_newton<N1>(ctx, a, w, max_it, rtol, resid, it_done, r0, keep_iterate ? FINISH_NONE : finish);
+      if (rc != FEDG_OK) return rc;
+      // the variables the solve has not finished
+      TendStore ts{};
+      for (int v = 0; v < 5; ++v) {
+        if (a.finish && v != VU && v != VV) continue;
+        const int u = ts.nv++;
+        ts.T[u] = tend[v];
+        ts.p[u] = w->pv[v];
+        ts.qs[u] = q[v];
+        ts.q[u] = a.qst[v];
+        ts.var0[u] = a.var0[v];
+        ts.varTmp[u] = a.varTmp[v];
       }
-      hipLaunchKernelGGL(hevi_tend_kernel, dim3((n + bs - 1) / bs), dim3(bs), 0, ctx->stream, tend[VD], tend[VT],
-                         tend[VW], tend[VU], tend[VV], w->pv[VD], w->pv[VT], w->pv[VW], w->pv[VU], w->pv[VV], q[VD],
-                         q[VT], q[VW], q[VU], q[VV], impl_fac, n);
+      ts.impl_fac = impl_fac;
+      ts.finish = finish;
+      const int bs = 256;
+      hipLaunchKernelGGL(hevi_tend_store_kernel, dim3((n + bs - 1) / bs), dim3(bs), 0, ctx->stream, ts, n);
       FEDG_HIP_CHECK(hipGetLastError());
       return FEDG_OK;
     }
