@@ -1334,15 +1334,14 @@ enum { TRC_TEND = 0, TRC_FCT = 1 };
 // node in order by one thread.
 // FLAT: the flat-terrain uniform box the context detected (Gsqrt = GsqrtH = 1,
 // GI3 = 0, axis-aligned unit normals, Escale and Fscale constant per
-// direction and face, the box's own face map): the same expressions with those
-// exact constants in place of the loads, and the face nodes formed
-// arithmetically except where the neighbour is the halo.
+// direction and face): the same expressions with those exact constants in
+// place of the loads.
 // Bound: HBM traffic (the tendency 41 KB per element at p = 7, the coefficient
 // 45) behind a chain of gathers, barriers and ordered sums.  The sums' terms
 // are multiplied by the threads that form them; the tendency's line
 // contractions run beside its face sums, the coefficient's mass sum beside
-// its.  48 x 48 x 16 elements at p = 7: tendency 481 -> 468 us, coefficient 449
-// -> 439 us (3.9 TB/s).
+// its.  48 x 48 x 16 elements at p = 7: coefficient 449 -> 444 us (3.9 TB/s), the
+// tendency 479 us as before.
 template <int N1, int EPB, int KIND, bool FLAT>
 __global__ void __launch_bounds__(EPB * N1 * N1 * N1) __attribute__((amdgpu_waves_per_eu(N1 >= 6 ? 8 : 4)))
 trcadv_kernel(const DevMesh m, const TrcArgs a) {
@@ -1376,12 +1375,6 @@ trcadv_kernel(const DevMesh m, const TrcArgs a) {
   if constexpr (TEND)
     for (int t = tid; t < N1 * N1; t += blockDim.x) sDt[(t % N1) * N1 + t / N1] = m.D1D[t];
   const int ke2d = FLAT || !valid ? 0 : m.EMap3Dto2D[ke];
-  [[maybe_unused]] int ei = 0, ej = 0, ek = 0;
-  if constexpr (FLAT) {
-    ei = ke % m.NeX;
-    ej = (ke / m.NeX) % m.NeY;
-    ek = ke / (m.NeX * m.NeY);
-  }
   if (valid) {
 #pragma unroll
     for (int u = 0; u < NFT; ++u) {
@@ -1389,25 +1382,7 @@ trcadv_kernel(const DevMesh m, const TrcArgs a) {
       if (fp >= NfpTot) break;
       const uint32_t gf = (uint32_t)fp + (uint32_t)NfpTot * ke;
       const int f = fp / Nfp, an = fp - f * Nfp;
-      uint32_t iM, iP;
-      if constexpr (FLAT) {
-        constexpr int opp[6] = {2, 3, 0, 1, 5, 4};
-        iM = (uint32_t)Np * ke + face_node<N1>(f, an);
-        int step = 0;  // to the neighbour's element
-        bool out = false;
-        switch (f) {
-          case 0: out = ej == 0; step = -m.NeX; break;
-          case 1: out = ei == m.NeX - 1; step = 1; break;
-          case 2: out = ej == m.NeY - 1; step = m.NeX; break;
-          case 3: out = ei == 0; step = -1; break;
-          case 4: out = ek == 0; step = -m.NeX * m.NeY; break;
-          default: out = ek == m.NeZ - 1; step = m.NeX * m.NeY; break;
-        }
-        iP = out ? (uint32_t)m.vmapP[gf] : (uint32_t)Np * (ke + step) + face_node<N1>(opp[f], an);
-      } else {
-        iM = (uint32_t)m.vmapM[gf];
-        iP = (uint32_t)m.vmapP[gf];
-      }
+      const uint32_t iM = (uint32_t)m.vmapM[gf], iP = (uint32_t)m.vmapP[gf];
       const double GsH = FLAT ? 1.0 : ldg(m.GsqrtH, (uint32_t)(face_node<N1>(f, an) % Nfp) + (uint32_t)Nfp * ke2d);
       const double Gsqrt_M = FLAT ? 1.0 : ldg(m.Gsqrt, iM), Gsqrt_P = FLAT ? 1.0 : ldg(m.Gsqrt, iP);
       const double GsqrtV_M = Gsqrt_M / GsH, GsqrtV_P = Gsqrt_P / GsH;
