@@ -44,12 +44,70 @@ enum { MODE_DROPIN = 0, MODE_FUSED_GENERAL = 1, MODE_FUSED_FLAT = 2, MODE_DROPIN
 // entries per element (24 KB at p = 7).
 template <int N1>
 __device__ __forceinline__ double lift_entry(const DevMesh& m, int f, int i, int j, int k) {
-  if (m.lift_tensor) return ldg(m.liftT, (uint32_t)((f >= 4 ? k : f == 1 || f == 3 ? i : j) + N1 * f));
+  if (N1 > 3 && m.lift_tensor) return ldg(m.liftT, (uint32_t)((f >= 4 ? k : f == 1 || f == 3 ? i : j) + N1 * f));
   return ldg(m.Lift, (uint32_t)(i + N1 * (j + N1 * k) + f * (N1 * N1 * N1)));
 }
 
-// Element kernel of every order and mode: EPB elements per workgroup, one
-// thread per node.  FM (drop-in modes; MODE_FUSED_FLAT always): the flat-terrain
+// Pointwise fluxes of variable v at a node (FDS/..._rhot_heve.F90:376-418).
+template <bool HEVI>
+__device__ __forceinline__ void point_flux(int v, const double (&q)[5], double Gs, double g13, double g23, double RGsqrtV,
+                                           double RDENS, double Th, double DP, double& f0, double& f1, double& f2) {
+  const double m0 = Gs * q[VU];
+  const double m1 = Gs * q[VV];
+  const double m2 = Gs * (q[VW] * RGsqrtV + g13 * q[VU] + g23 * q[VV]);
+  if (v == VD) {
+    f0 = m0;
+    f1 = m1;
+    f2 = m2;
+  } else if (v == VT) {
+    const double pt_ = (Th + q[VT]) * RDENS;
+    f0 = m0 * pt_;
+    f1 = m1 * pt_;
+    f2 = m2 * pt_;
+  } else if (v == VW) {
+    const double w_ = q[VW] * RDENS;
+    f0 = m0 * w_;
+    f1 = m1 * w_;
+    f2 = HEVI ? m2 * w_ : m2 * w_ + Gs * DP * RGsqrtV;
+  } else if (v == VU) {
+    const double GsqrtDPRES_ = Gs * DP;
+    const double u_ = q[VU] * RDENS;
+    f0 = m0 * u_ + GsqrtDPRES_;
+    f1 = m1 * u_;
+    f2 = m2 * u_ + GsqrtDPRES_ * g13;
+  } else {
+    const double GsqrtDPRES_ = Gs * DP;
+    const double v_ = q[VV] * RDENS;
+    f0 = m0 * v_;
+    f1 = m1 * v_ + GsqrtDPRES_;
+    f2 = m2 * v_ + GsqrtDPRES_ * g23;
+  }
+}
+
+// Exterior node of face node a (own node pm) of face f of element (ei, ej, ek)
+// of the flat box: its element level and node; true at a closed boundary,
+// where it is the own node.
+template <int N1>
+__device__ __forceinline__ bool flat_exterior(const DevMesh& m, int ei, int ej, int ek, int f, int a, int pm, int& ni,
+                                              int& nj, int& nk, int& nodeP) {
+  ni = ei, nj = ej, nk = ek;
+  bool closed = false;
+  switch (f) {
+    case 0: nj -= 1; if (nj < 0) { if (m.periodic[1]) nj = m.NeY - 1; else closed = true; } break;
+    case 1: ni += 1; if (ni >= m.NeX) { if (m.periodic[0]) ni = 0; else closed = true; } break;
+    case 2: nj += 1; if (nj >= m.NeY) { if (m.periodic[1]) nj = 0; else closed = true; } break;
+    case 3: ni -= 1; if (ni < 0) { if (m.periodic[0]) ni = m.NeX - 1; else closed = true; } break;
+    case 4: nk -= 1; if (nk < 0) { if (m.periodic[2]) nk = m.NeZ - 1; else closed = true; } break;
+    default: nk += 1; if (nk >= m.NeZ) { if (m.periodic[2]) nk = 0; else closed = true; } break;
+  }
+  constexpr int opp[6] = {2, 3, 0, 1, 5, 4};
+  nodeP = closed ? pm : face_node<N1>(opp[f], a);
+  if (closed) ni = ei, nj = ej, nk = ek;
+  return closed;
+}
+
+// Element kernel, face sides from memory: EPB elements per workgroup, one thread
+// per node.  FM (drop-in modes; MODE_FUSED_FLAT always): the flat-terrain
 // uniform box the context detected, whose metric arrays hold Gsqrt = GsqrtH =
 // 1, GI3 = 0, axis-aligned unit normals and constant Escale and Fscale: those
 // values are taken as constants, every operation kept.
@@ -57,20 +115,19 @@ __device__ __forceinline__ double lift_entry(const DevMesh& m, int f, int i, int
 //    side's lines are the ones the element's own threads load), and the face
 //    flux needs no barrier; only the fluxes, the face jumps and DDENS go
 //    through LDS.
-//  - NB flux buffers: all five variables before one barrier at p = 3..5, two
-//    variables per barrier in four buffers elsewhere (as in heve7_body), where
-//    five would leave fewer workgroups per CU.
-//  - At most 128 VGPRs: four wavefronts per SIMD (the layout that staged the
-//    state in LDS and held every variable's RK operands took 140-226 and left
-//    two).
+//  - NB flux buffers: two and a barrier per variable at p = 3..5, where that
+//    lets one more element on a CU; elsewhere, and for the filter's two halves,
+//    four and two variables per barrier (as in heve7_body).
+//  - At p >= 5 every contraction is formed on the spot, so that the forms
+//    without physics tendencies stay at 128 VGPRs or below (four wavefronts per
+//    SIMD) without a spill.
 //  - The base state comes from the per-level tables where it is horizontally
 //    homogeneous (MODE_FUSED_FLAT), and the RK operands are all loaded before
 //    the first barrier.
+//  - Stage results are stored with the non-temporal hint where the boxes these
+//    orders are run on outgrow the caches (p >= 6).
 // Bound: HBM traffic and the latency of a chain of loads, barriers and LDS
-// round trips, as the p = 7 stage kernel.  Measured against the layout before:
-// RK4 step at p = 5, 41 x 37 x 13 elements 1.64 -> 1.28 ms; p = 7 over terrain,
-// 27 x 19 x 11 1.46 -> 1.00 ms; drop-in right-hand side at p = 7, 40 x 32 x 16
-// 1.19 -> 0.74 ms (of it 1.01 -> 0.56 ms the tendency).
+// round trips, as the p = 7 stage kernel.
 // KIND (fused modes): STAGE_PHYS, physics tendencies join the stage's tendency
 // (a kernel of its own because their power keeps registers from everything
 // else); STAGE_FILTER, the step's last stage with the modal filter applied to
@@ -80,7 +137,7 @@ __device__ __forceinline__ double lift_entry(const DevMesh& m, int f, int i, int
 // elements: 66.8 -> 60.1 us).
 enum { STAGE_PLAIN = 0, STAGE_PHYS = 1, STAGE_FILTER = 2 };
 template <int N1, int EPB, int MODE, bool FM, int KIND = STAGE_PLAIN>
-__global__ void __launch_bounds__(EPB* N1* N1* N1) __attribute__((amdgpu_waves_per_eu(KIND == STAGE_PHYS ? 2 : 4)))
+__global__ void __launch_bounds__(EPB* N1* N1* N1) __attribute__((amdgpu_waves_per_eu(KIND == STAGE_PHYS || N1 <= 5 ? 2 : 4)))
 heve_kernel(const DevMesh m, const Consts c, const TendIn in, const RkOut rk) {
   constexpr int Np = N1 * N1 * N1, Nfp = N1 * N1, NfpTot = 6 * Nfp;
   constexpr bool HEVI = MODE == MODE_DROPIN_HEVI;
@@ -89,13 +146,22 @@ heve_kernel(const DevMesh m, const Consts c, const TendIn in, const RkOut rk) {
   constexpr bool FLAT = MODE == MODE_FUSED_FLAT;  // neighbours formed arithmetically
   constexpr bool FUSED = !DROPIN;
   static_assert(!FLAT || FM, "the arithmetic neighbours are those of the flat box");
-  constexpr int NB = N1 >= 4 && N1 <= 6 ? 5 : 4;
+  constexpr int NB = N1 >= 4 && N1 <= 6 && KIND != STAGE_FILTER && !(N1 == 4 && !FM) ? 2 : 4;
+  // pow tables in LDS, except where they would be a large part of a workgroup's loads
+  constexpr bool POW_LDS = FUSED && N1 >= 5;
+  // non-temporal hint on what is streamed once
+  constexpr bool NT = N1 >= 7 || (N1 == 6 && DROPIN);
+  auto load_once = [](const double* b, uint32_t x) { return NT ? ldg_nt(b, x) : ldg(b, x); };
+  auto store_once = [](double* b, uint32_t x, double y) {
+    if constexpr (NT) stg_nt(b, x, y);
+    else stg(b, x, y);
+  };
   __shared__ double sDt[N1 * N1];
   __shared__ double sI[N1 * N1];
   __shared__ double sRho[EPB][Np];
   __shared__ double sF[NB][EPB][3][Np];
   __shared__ double sDF[EPB][5][CCO ? 1 : NfpTot];
-  __shared__ double sPow[FUSED ? 640 : 1];
+  __shared__ double sPow[POW_LDS ? 640 : 1];
   constexpr bool PHYS = KIND == STAGE_PHYS, FILTER = KIND == STAGE_FILTER;
   static_assert(FUSED || KIND == STAGE_PLAIN, "");
 
@@ -110,7 +176,11 @@ heve_kernel(const DevMesh m, const Consts c, const TendIn in, const RkOut rk) {
     sDt[(t % N1) * N1 + t / N1] = m.D1D[t];
     sI[t] = m.Itr[t];
   }
-  if constexpr (FUSED) pow_tables_to(sPow, tid, EPB * Np);
+  if constexpr (POW_LDS) pow_tables_to(sPow, tid, EPB * Np);
+  auto dpres = [&](double DT, double Thyd, double Phyd, double Rt, double Cv, double Cp) {
+    if constexpr (POW_LDS) return dpres_of_tab(DT, Thyd, Phyd, Rt, Cv, Cp, c, sPow);
+    else return dpres_of(DT, Thyd, Phyd, Rt, Cv, Cp, c);
+  };
 
   // base state: full fields, or (MODE_FUSED_FLAT) the per-level tables
   const bool lvl = FLAT && in.lvl != nullptr;
@@ -178,27 +248,9 @@ heve_kernel(const DevMesh m, const Consts c, const TendIn in, const RkOut rk) {
     if constexpr (DROPIN) {
       iP = hP = (uint32_t)m.vmapP[gf];
     } else if constexpr (FLAT) {
-      int ni = ei, nj = ej, nk = ek;
-      bool closed = false;
-      switch (f) {
-        case 0: nj -= 1; if (nj < 0) { if (m.periodic[1]) nj = m.NeY - 1; else closed = true; } break;
-        case 1: ni += 1; if (ni >= m.NeX) { if (m.periodic[0]) ni = 0; else closed = true; } break;
-        case 2: nj += 1; if (nj >= m.NeY) { if (m.periodic[1]) nj = 0; else closed = true; } break;
-        case 3: ni -= 1; if (ni < 0) { if (m.periodic[0]) ni = m.NeX - 1; else closed = true; } break;
-        case 4: nk -= 1; if (nk < 0) { if (m.periodic[2]) nk = m.NeZ - 1; else closed = true; } break;
-        default: nk += 1; if (nk >= m.NeZ) { if (m.periodic[2]) nk = 0; else closed = true; } break;
-      }
-      int nodeP = pm;
-      iP = (uint32_t)Np * ke;
-      if (closed) {
-        nk = ek;
-        bc = m.bnd_bc[f];
-      } else {
-        constexpr int opp[6] = {2, 3, 0, 1, 5, 4};
-        nodeP = face_node<N1>(opp[f], a);
-        iP = (uint32_t)Np * (ni + m.NeX * (nj + m.NeY * nk));
-      }
-      iP += nodeP;
+      int ni, nj, nk, nodeP;
+      if (flat_exterior<N1>(m, ei, ej, ek, f, a, pm, ni, nj, nk, nodeP)) bc = m.bnd_bc[f];
+      iP = (uint32_t)Np * (ni + m.NeX * (nj + m.NeY * nk)) + nodeP;
       hM = lvl ? (uint32_t)(Np * ek + pm) : iM;
       hP = lvl ? (uint32_t)(Np * nk + nodeP) : iP;
     } else {
@@ -244,23 +296,11 @@ heve_kernel(const DevMesh m, const Consts c, const TendIn in, const RkOut rk) {
     for (int v = 0; v < 5; ++v) sDF[e][v][fp] = df[v];
   };
   if (valid && !CCO) {
-    if constexpr (NfpTot > Np && NfpTot <= 2 * Np) {
-      // two face nodes for some threads (p = 2..4): the second's loads issued
-      // with the first's, one latency instead of two
-      Side M, P, M2, P2;
-      const int fp2 = p + Np;
-      int bc2 = FEDG_BND_NONE;
-      const int bc = load_face(p, M, P);
-      if (fp2 < NfpTot) bc2 = load_face(fp2, M2, P2);
-      face_flux(p, bc, M, P);
-      if (fp2 < NfpTot) face_flux(fp2, bc2, M2, P2);
-    } else {
 #pragma unroll 1
-      for (int fp = p; fp < NfpTot; fp += Np) {
-        Side M, P;
-        const int bc = load_face(fp, M, P);
-        face_flux(fp, bc, M, P);
-      }
+    for (int fp = p; fp < NfpTot; fp += Np) {
+      Side M, P;
+      const int bc = load_face(fp, M, P);
+      face_flux(fp, bc, M, P);
     }
   }
   __builtin_amdgcn_sched_barrier(0);
@@ -276,39 +316,9 @@ heve_kernel(const DevMesh m, const Consts c, const TendIn in, const RkOut rk) {
     for (int f = 0; f < 6; ++f) L[f] = lift_entry<N1>(m, f, i, j, k);
   }
 
-  // pointwise fluxes of a variable (FDS/..._rhot_heve.F90:376-418)
   auto put_flux = [&](int v) {
-    const double m0 = Gs * q[VU];
-    const double m1 = Gs * q[VV];
-    const double m2 = Gs * (q[VW] * RGsqrtV + g13 * q[VU] + g23 * q[VV]);
     double f0, f1, f2;
-    if (v == VD) {
-      f0 = m0;
-      f1 = m1;
-      f2 = m2;
-    } else if (v == VT) {
-      const double pt_ = (Th + q[VT]) * RDENS;
-      f0 = m0 * pt_;
-      f1 = m1 * pt_;
-      f2 = m2 * pt_;
-    } else if (v == VW) {
-      const double w_ = q[VW] * RDENS;
-      f0 = m0 * w_;
-      f1 = m1 * w_;
-      f2 = HEVI ? m2 * w_ : m2 * w_ + Gs * DP * RGsqrtV;
-    } else if (v == VU) {
-      const double GsqrtDPRES_ = Gs * DP;
-      const double u_ = q[VU] * RDENS;
-      f0 = m0 * u_ + GsqrtDPRES_;
-      f1 = m1 * u_;
-      f2 = m2 * u_ + GsqrtDPRES_ * g13;
-    } else {
-      const double GsqrtDPRES_ = Gs * DP;
-      const double v_ = q[VV] * RDENS;
-      f0 = m0 * v_;
-      f1 = m1 * v_ + GsqrtDPRES_;
-      f2 = m2 * v_ + GsqrtDPRES_ * g23;
-    }
+    point_flux<HEVI>(v, q, Gs, g13, g23, RGsqrtV, RDENS, Th, DP, f0, f1, f2);
     const int b = v % NB;
     sF[b][e][0][p] = f0;
     sF[b][e][1][p] = f1;
@@ -323,8 +333,8 @@ heve_kernel(const DevMesh m, const Consts c, const TendIn in, const RkOut rk) {
     Ops op{0.0, 0.0, 0.0, 0.0, 0.0};
     if (!valid) return op;
     if constexpr (FUSED) {
-      if (rk.mode == 1) op.rA = ldg_nt(rk.var0[v], o);
-      if (rk.mode == 1 || rk.mode == 2) op.rB = ldg_nt(rk.varTmp[v], o);
+      if (rk.mode == 1) op.rA = load_once(rk.var0[v], o);
+      if (rk.mode == 1 || rk.mode == 2) op.rB = load_once(rk.varTmp[v], o);
       if (v == VT) op.Ph = ldg(PRES_hyd, oh);
     }
     if (v == VU || v == VV) {
@@ -421,11 +431,11 @@ heve_kernel(const DevMesh m, const Consts c, const TendIn in, const RkOut rk) {
       double qn;
       switch (rk.mode) {
         case 0:
-          stg_nt(rk.varTmp[v], o, q[v] + rk.cb * T);
+          store_once(rk.varTmp[v], o, q[v] + rk.cb * T);
           qn = q[v] + rk.ca * T;
           break;
         case 1:
-          stg_nt(rk.varTmp[v], o, cur.rB + rk.cb * T);
+          store_once(rk.varTmp[v], o, cur.rB + rk.cb * T);
           qn = cur.rA + rk.ca * T;
           break;
         case 2:
@@ -439,20 +449,19 @@ heve_kernel(const DevMesh m, const Consts c, const TendIn in, const RkOut rk) {
         qf[v] = qn;
         return;
       }
-      stg_nt(rk.out[v], o, qn);
+      store_once(rk.out[v], o, qn);
       // pressure perturbation of the new state, read by the next stage (own
       // node and the neighbours' face nodes) instead of recomputed
-      if (v == VT) stg_nt(rk.DPout, o, dpres_of_tab(qn, Th, cur.Ph, Rt, Cv, Cp, c, sPow));
+      if (v == VT) store_once(rk.DPout, o, dpres(qn, Th, cur.Ph, Rt, Cv, Cp));
     } else {
-      stg_nt(rk.out[v], o, T);
+      store_once(rk.out[v], o, T);
     }
   };
-  if constexpr (NB == 5) {
-#pragma unroll
-    for (int v = 0; v < 5; ++v) put_flux(v);
-    __syncthreads();
+  if constexpr (NB == 2) {
 #pragma unroll
     for (int v = 0; v < 5; ++v) {
+      put_flux(v);
+      __syncthreads();
       update(v);
       // one variable's operands at a time, or every variable's stay live
       __builtin_amdgcn_sched_barrier(0);
@@ -520,7 +529,7 @@ heve_kernel(const DevMesh m, const Consts c, const TendIn in, const RkOut rk) {
 #pragma unroll
       for (int l = 1; l < N1; ++l) x = x + a[Nfp * l] * h[l];
       x = x * RGsqrt;
-      stg_nt(rk.out[v], o, x);
+      store_once(rk.out[v], o, x);
       if (v == VT) {
         double Rt = c.Rdry, Cv = c.CVdry, Cp = c.CPdry;
         if (in.Rtot != nullptr) {
@@ -528,15 +537,363 @@ heve_kernel(const DevMesh m, const Consts c, const TendIn in, const RkOut rk) {
           Cv = ldg(in.CVtot, o);
           Cp = ldg(in.CPtot, o);
         }
-        stg_nt(rk.DPout, o, dpres_of_tab(x, Th, ops[VT].Ph, Rt, Cv, Cp, c, sPow));
+        store_once(rk.DPout, o, dpres(x, Th, ops[VT].Ph, Rt, Cv, Cp));
       }
     }
   }
 }
 
-// own-node values staged in LDS by heve32_kernel: DDENS, DRHOT, MOMZ, MOMX,
-// MOMY (VID order), then DENS_hyd, PRES_hyd, THERM_hyd, DPRES
+// own-node values staged in LDS by heve_staged_kernel and heve32_kernel:
+// DDENS, DRHOT, MOMZ, MOMX, MOMY (VID order), then DENS_hyd, PRES_hyd,
+// THERM_hyd, DPRES
 enum { S_DH = 5, S_PH = 6, S_TH = 7, S_DP = 8, S_N = 9 };
+
+// Element kernel, own state staged in LDS: the layout for low orders and small
+// meshes (staged_element_kernel).  The interior side of a face node comes
+// from LDS, one variable's fluxes are in work at a time in two buffers, and
+// the derivative matrix's rows stay in registers.  At low orders an element
+// has as many face nodes as nodes or more, and loading their interior sides
+// costs more than the registers this layout takes (132-162 VGPRs, three
+// wavefronts per SIMD at p = 2, 3); on small meshes one workgroup has the CU to
+// itself and the rows read again from LDS for every variable are what it waits
+// for.
+template <int N1, int EPB, int MODE>
+__global__ void __launch_bounds__(EPB * N1 * N1 * N1, 2)
+heve_staged_kernel(const DevMesh m, const Consts c, const TendIn in, const RkOut rk) {
+  constexpr int Np = N1 * N1 * N1, Nfp = N1 * N1, NfpTot = 6 * Nfp;
+  constexpr bool HEVI = MODE == MODE_DROPIN_HEVI;
+  constexpr bool CCO = MODE == MODE_DROPIN_CCO;
+  constexpr bool DROPIN = MODE == MODE_DROPIN || HEVI || CCO;
+  constexpr bool FLAT = MODE == MODE_FUSED_FLAT;
+  constexpr bool FUSED = !DROPIN;
+  // exterior values are loaded before the first barrier when every face node
+  // has its own thread (p >= 5); otherwise inside the face loop
+  constexpr bool PRELOAD = NfpTot <= Np;
+
+  __shared__ double sDt[N1 * N1];
+  __shared__ double sI[N1 * N1];
+  __shared__ double sS[EPB][S_N][Np];
+  __shared__ double sF[2][EPB][3][Np];
+  __shared__ double sDF[EPB][5][NfpTot];
+
+  const int tid = threadIdx.x;
+  const int e = tid / Np;
+  const int p = tid - e * Np;
+  int blk = blockIdx.x;
+  if constexpr (FLAT) blk = xcd_remap(blk, gridDim.x);
+  const int ke = blk * EPB + e;
+  const bool valid = ke < m.Ne;
+  const int i = p % N1, j = (p / N1) % N1, k = p / Nfp;
+  const double gamm = c.CPdry / c.CVdry;
+
+  for (int t = tid; t < N1 * N1; t += blockDim.x) {
+    sDt[(t % N1) * N1 + t / N1] = m.D1D[t];
+    sI[t] = m.Itr[t];
+  }
+
+  // ---- exterior side of this thread's face node: index and boundary kind ----
+  const int fp0 = p;
+  const int f0 = fp0 / Nfp, a0 = fp0 - f0 * Nfp;
+  const bool has_face = valid && fp0 < NfpTot;
+  uint32_t iP0 = 0;
+  int bc0 = FEDG_BND_NONE;
+  const int pm0 = face_node<N1>(f0 < 6 ? f0 : 0, a0);
+  auto exterior = [&](int f, int a, int pm, uint32_t& iP, int& bc) {
+    const uint32_t gf = (uint32_t)(f * Nfp + a) + (uint32_t)NfpTot * ke;
+    if constexpr (DROPIN) {
+      iP = (uint32_t)m.vmapP[gf];
+      bc = FEDG_BND_NONE;
+    } else if constexpr (FLAT) {
+      int ni, nj, nk, nodeP;
+      bc = flat_exterior<N1>(m, ke % m.NeX, (ke / m.NeX) % m.NeY, ke / (m.NeX * m.NeY), f, a, pm, ni, nj, nk, nodeP)
+               ? m.bnd_bc[f]
+               : FEDG_BND_NONE;
+      iP = (uint32_t)Np * (ni + m.NeX * (nj + m.NeY * nk)) + nodeP;
+    } else {
+      iP = (uint32_t)m.nbr[gf];
+      bc = m.nbr_bc[gf];
+    }
+  };
+  struct Ext {
+    double DD, DT, MZ, MX, MY, Dh, Ph, Th, DP, Gs, g13, g23;
+  };
+  auto load_ext = [&](uint32_t iP, Ext& x) {
+    x.DD = ldg(in.q[VD], iP); x.DT = ldg(in.q[VT], iP); x.MZ = ldg(in.q[VW], iP);
+    x.MX = ldg(in.q[VU], iP); x.MY = ldg(in.q[VV], iP);
+    x.Dh = ldg(in.DENS_hyd, iP); x.Ph = ldg(in.PRES_hyd, iP); x.Th = ldg(in.THERM_hyd, iP);
+    x.DP = ldg(in.DPRES, iP);
+    if constexpr (!FLAT) {
+      x.Gs = ldg(m.Gsqrt, iP); x.g13 = ldg(m.G13, iP); x.g23 = ldg(m.G23, iP);
+    } else {
+      x.Gs = 1.0; x.g13 = 0.0; x.g23 = 0.0;
+    }
+  };
+  Ext X0;
+  if constexpr (PRELOAD && !CCO) {
+    if (has_face) {
+      exterior(f0, a0, pm0, iP0, bc0);
+      load_ext(iP0, X0);
+    }
+  }
+
+  // ---- own node: state, base state, pressure ----
+  const uint32_t o = (uint32_t)Np * (valid ? ke : 0) + p;
+  double q[5] = {0, 0, 0, 0, 0};
+  double Dh = 0, Ph = 0, Th = 0, DP = 0;
+  double Gs = 1.0, g13 = 0.0, g23 = 0.0, GsH = 1.0;
+  int ke2d = 0;
+  double cor = 0.0, dpx = 0.0, dpy = 0.0;
+  if (valid) {
+#pragma unroll
+    for (int v = 0; v < 5; ++v) q[v] = ldg(in.q[v], o);
+    Dh = ldg(in.DENS_hyd, o);
+    Ph = ldg(in.PRES_hyd, o);
+    Th = ldg(in.THERM_hyd, o);
+    if constexpr (FLAT) {
+      ke2d = ke % (m.NeX * m.NeY);
+    } else {
+      Gs = ldg(m.Gsqrt, o);
+      g13 = ldg(m.G13, o);
+      g23 = ldg(m.G23, o);
+      ke2d = m.EMap3Dto2D[ke];
+      GsH = ldg(m.GsqrtH, (uint32_t)(i + N1 * j) + (uint32_t)Nfp * ke2d);
+    }
+    cor = ldg(in.CORIOLIS, (uint32_t)(i + N1 * j) + (uint32_t)Nfp * ke2d);
+    dpx = ldg(in.DPhydDx, o);
+    dpy = ldg(in.DPhydDy, o);
+    DP = ldg(in.DPRES, o);
+  }
+  double L[6] = {0, 0, 0, 0, 0, 0};
+  if constexpr (!CCO) {
+#pragma unroll
+    for (int f = 0; f < 6; ++f) L[f] = ldg(m.Lift, (uint32_t)(p + f * Np));
+  }
+#pragma unroll
+  for (int v = 0; v < 5; ++v) sS[e][v][p] = q[v];
+  sS[e][S_DH][p] = Dh;
+  sS[e][S_PH][p] = Ph;
+  sS[e][S_TH][p] = Th;
+  sS[e][S_DP][p] = DP;
+  __syncthreads();
+
+  // ---- face phase: Rusanov flux at the element's face nodes ----
+  if (valid && !CCO) {
+    for (int fp = p; fp < NfpTot; fp += Np) {
+      const int f = fp / Nfp, a = fp - f * Nfp;
+      const int pm = PRELOAD ? pm0 : face_node<N1>(f, a);
+      const uint32_t gf = (uint32_t)fp + (uint32_t)NfpTot * ke;
+      uint32_t iP;
+      int bc;
+      Ext X;
+      if constexpr (PRELOAD) {
+        iP = iP0;
+        bc = bc0;
+        X = X0;
+      } else {
+        exterior(f, a, pm, iP, bc);
+        load_ext(iP, X);
+      }
+      const uint32_t iM = DROPIN ? (uint32_t)m.vmapM[gf] : (uint32_t)Np * ke + pm;
+      const int pmM = DROPIN ? (int)(iM - (uint32_t)Np * ke) : pm;
+      Side M, P;
+      double nx, ny, nz, Fs;
+      if constexpr (FLAT) {
+        nx = (f == 1) ? 1.0 : (f == 3) ? -1.0 : 0.0;
+        ny = (f == 2) ? 1.0 : (f == 0) ? -1.0 : 0.0;
+        nz = (f == 5) ? 1.0 : (f == 4) ? -1.0 : 0.0;
+        Fs = m.fF[f];
+        M.Gsqrt = 1.0; M.G13 = 0.0; M.G23 = 0.0;
+      } else {
+        nx = ldg(m.nx, gf);
+        ny = ldg(m.ny, gf);
+        nz = ldg(m.nz, gf);
+        Fs = ldg(m.Fscale, gf);
+        M.Gsqrt = ldg(m.Gsqrt, iM); M.G13 = ldg(m.G13, iM); M.G23 = ldg(m.G23, iM);
+      }
+      if (DROPIN && (uint32_t)pmM >= (uint32_t)Np) {
+        // a map whose interior node lies in another element
+        M.DD = ldg(in.q[VD], iM); M.DT = ldg(in.q[VT], iM); M.MZ = ldg(in.q[VW], iM);
+        M.MX = ldg(in.q[VU], iM); M.MY = ldg(in.q[VV], iM);
+        M.Dhyd = ldg(in.DENS_hyd, iM); M.Phyd = ldg(in.PRES_hyd, iM); M.Thyd = ldg(in.THERM_hyd, iM);
+        M.DP = ldg(in.DPRES, iM);
+      } else {
+        M.DD = sS[e][VD][pmM]; M.DT = sS[e][VT][pmM]; M.MZ = sS[e][VW][pmM];
+        M.MX = sS[e][VU][pmM]; M.MY = sS[e][VV][pmM];
+        M.Dhyd = sS[e][S_DH][pmM]; M.Phyd = sS[e][S_PH][pmM]; M.Thyd = sS[e][S_TH][pmM];
+        M.DP = sS[e][S_DP][pmM];
+      }
+      P.Gsqrt = X.Gs; P.G13 = X.g13; P.G23 = X.g23;
+      P.DD = X.DD; P.DT = X.DT; P.MZ = X.MZ; P.MX = X.MX; P.MY = X.MY;
+      P.Dhyd = X.Dh; P.Phyd = X.Ph; P.Thyd = X.Th;
+      P.DP = X.DP;
+      if (bc != FEDG_BND_NONE) {
+        // exterior momentum from the interior node, as applyBC writes it into the halo
+        double GH = 1.0, g11 = 1.0, g12 = 0.0, g22 = 1.0;
+        if constexpr (!FLAT) {
+          const uint32_t h = (uint32_t)(pm % Nfp) + (uint32_t)Nfp * m.EMap3Dto2D[ke];
+          GH = ldg(m.GsqrtH, h);
+          g11 = ldg(m.G11, h);
+          g12 = ldg(m.G12, h);
+          g22 = ldg(m.G22, h);
+        }
+        reflect_momentum(bc, M.Gsqrt, GH, g11, g12, g22, M.G13, M.G23, nx, ny, nz, M.MX, M.MY, M.MZ, P.MX, P.MY,
+                         P.MZ);
+      }
+      double df[5];
+      if constexpr (HEVI) rusanov_hevi(M, P, nx, ny, nz, Fs, gamm, df);
+      else rusanov(M, P, nx, ny, nz, Fs, gamm, df);
+#pragma unroll
+      for (int v = 0; v < 5; ++v) sDF[e][v][fp] = df[v];
+    }
+  }
+
+  // ---- volume phase ----
+  // RK operands, loaded now so their latency overlaps the contractions
+  double rkA[5] = {0, 0, 0, 0, 0}, rkB[5] = {0, 0, 0, 0, 0};
+  if constexpr (FUSED) {
+    if (valid) {
+      if (rk.mode == 1) {
+#pragma unroll
+        for (int v = 0; v < 5; ++v) {
+          rkA[v] = ldg(rk.var0[v], o);
+          rkB[v] = ldg(rk.varTmp[v], o);
+        }
+      } else if (rk.mode == 2) {
+#pragma unroll
+        for (int v = 0; v < 5; ++v) rkB[v] = ldg(rk.varTmp[v], o);
+      }
+    }
+  }
+  const double RDENS = 1.0 / (q[VD] + Dh);
+  const double GsqrtV = Gs / GsH;
+  const double RGsqrtV = 1.0 / GsqrtV;
+  const double RGsqrt = 1.0 / Gs;
+  double E11, E22, E33;
+  if constexpr (FLAT) {
+    E11 = m.fE[0];
+    E22 = m.fE[1];
+    E33 = m.fE[2];
+  } else {
+    E11 = valid ? ldg(m.E11, o) : 0.0;
+    E22 = valid ? ldg(m.E22, o) : 0.0;
+    E33 = valid ? ldg(m.E33, o) : 0.0;
+  }
+  // VFilterPM1 of DDENS (ELM/..._tensorprod3D.F90:2828-2839)
+  double drho = sS[e][VD][i + N1 * j] * sI[N1 * k];
+#pragma unroll
+  for (int l = 1; l < N1; ++l) drho = drho + sS[e][VD][i + N1 * (j + N1 * l)] * sI[l + N1 * k];
+
+  // One variable at a time: pointwise flux, Div_var5
+  // (ELM/..._tensorprod3D.F90:2760-2783: Dx Fx, Dy Fy, Dz Fz and the lift of
+  // del_flux), tendency (FDS/..._rhot_heve.F90:424-483) and its RK update
+  // (CMN/scale_timeint_rk.F90:2232-2350 with one tendency buffer).
+#pragma unroll
+  for (int v = 0; v < 5; ++v) {
+    double f0, f1, f2;
+    point_flux<HEVI>(v, q, Gs, g13, g23, RGsqrtV, RDENS, Th, DP, f0, f1, f2);
+    const int b = v & 1;
+    sF[b][e][0][p] = f0;
+    sF[b][e][1][p] = f1;
+    sF[b][e][2][p] = f2;
+    __syncthreads();
+    const double* Fx = sF[b][e][0];
+    const double* Fy = sF[b][e][1];
+    const double* Fz = sF[b][e][2];
+    // one direction at a time, so that only one line of operands is live
+    // (sDt holds D1D transposed: row i of D1D is sDt[N1*i .. N1*i+N1-1])
+    double dx = sDt[N1 * i] * Fx[N1 * (j + N1 * k)];
+#pragma unroll
+    for (int l = 1; l < N1; ++l) dx = dx + sDt[l + N1 * i] * Fx[l + N1 * (j + N1 * k)];
+    __builtin_amdgcn_sched_barrier(0);
+    double dy = Fy[i + N1 * (N1 * k)] * sDt[N1 * j];
+#pragma unroll
+    for (int l = 1; l < N1; ++l) dy = dy + Fy[i + N1 * (l + N1 * k)] * sDt[l + N1 * j];
+    __builtin_amdgcn_sched_barrier(0);
+    double dz = Fz[i + N1 * j] * sDt[N1 * k];
+#pragma unroll
+    for (int l = 1; l < N1; ++l) dz = dz + Fz[i + N1 * (j + N1 * l)] * sDt[l + N1 * k];
+    __builtin_amdgcn_sched_barrier(0);
+    const double* dfv = sDF[e][v];
+    double X;
+    if constexpr (CCO) {
+      // Div_var5_2: the three line contractions only (..._rhot_heve.F90:607-669)
+      X = E11 * dx + E22 * dy + E33 * dz;
+    } else {
+      const double lift = L[0] * dfv[i + N1 * k] + L[1] * dfv[Nfp + j + N1 * k] + L[2] * dfv[2 * Nfp + i + N1 * k] +
+                          L[3] * dfv[3 * Nfp + j + N1 * k] + L[4] * dfv[4 * Nfp + i + N1 * j] +
+                          L[5] * dfv[5 * Nfp + i + N1 * j];
+      // HEVI: DENS and RHOT have no vertical flux term, MOMZ no buoyancy
+      X = (HEVI && (v == VD || v == VT)) ? E11 * dx + E22 * dy + lift : E11 * dx + E22 * dy + E33 * dz + lift;
+    }
+    double T;
+    if (v == VD || v == VT) {
+      T = -X * RGsqrt;
+    } else if (v == VW) {
+      T = HEVI ? -X * RGsqrt : -X * RGsqrt - c.GRAV * drho;
+    } else if (v == VU) {
+      T = -dpx + cor * q[VV];
+      T = T - X * RGsqrt;
+    } else {
+      T = -dpy - cor * q[VU];
+      T = T - X * RGsqrt;
+    }
+    if constexpr (FUSED) {
+      // add_phy_tend (FDS/scale_atm_dyn_dgm_driver_nonhydro3d.F90:1098-1178):
+      // the physics tendencies join the stage's tendency before the update
+      if (valid && in.tp[0] != nullptr) {
+        if (v == VT) {
+          double Rt = c.Rdry, Cv = c.CVdry, Cp = c.CPdry;
+          if (in.Rtot != nullptr) {
+            Rt = ldg(in.Rtot, o);
+            Cv = ldg(in.CVtot, o);
+            Cp = ldg(in.CPtot, o);
+          }
+          T = phys_add_rhot(T, ldg(in.tp[VT], o), ldg(in.tp[5], o), pres_of(q[VT], Th, Rt, Cv, Cp, c), Rt, Cp, c);
+        } else {
+          T = T + ldg(in.tp[v], o);
+        }
+      }
+    }
+    if (valid) {
+      if constexpr (DROPIN) {
+        stg(rk.out[v], o, T);
+      } else {
+        double qn;
+        switch (rk.mode) {
+          case 0:
+            stg(rk.varTmp[v], o, q[v] + rk.cb * T);
+            qn = q[v] + rk.ca * T;
+            break;
+          case 1:
+            stg(rk.varTmp[v], o, rkB[v] + rk.cb * T);
+            qn = rkA[v] + rk.ca * T;
+            break;
+          case 2:
+            qn = rkB[v] + rk.cb * T;
+            break;
+          default:
+            qn = q[v] + rk.cb * T;
+            break;
+        }
+        stg(rk.out[v], o, qn);
+        if (v == VT) {
+          // pressure perturbation of the new state, read by the next stage
+          // (own node and the neighbours' face nodes) instead of recomputed
+          double Rt = c.Rdry, Cv = c.CVdry, Cp = c.CPdry;
+          if (in.Rtot != nullptr) {
+            Rt = ldg(in.Rtot, o);
+            Cv = ldg(in.CVtot, o);
+            Cp = ldg(in.CPtot, o);
+          }
+          stg(rk.DPout, o, dpres_of(qn, Th, Ph, Rt, Cv, Cp, c));
+        }
+      }
+    }
+    // finish this variable before the next one's LDS traffic; otherwise the
+    // scheduler defers the arithmetic and every variable's operands stay live
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
 
 // ---------------------------------------------------------------------------
 // FP32 perturbation form of the fused HEVE stage (flat-terrain box, dry air).
@@ -1832,11 +2189,46 @@ constexpr int epb_for() {
   return (N1 * N1 * N1 >= 128) ? 1 : (256 / (N1 * N1 * N1));
 }
 
-// elements per workgroup of heve_kernel: two at p = 5, whose 216 nodes fill
-// 3.4 wavefronts alone and 6.75 of 7 in pairs
-template <int N1>
+// Elements per workgroup of heve_kernel: one from p = 4 on, whose 125 nodes fill
+// two wavefronts (a barrier then waits for one element; RK4 step at p = 5, 41 x
+// 37 x 13 elements, two with five flux buffers 1.27 ms, one with two 1.18 ms);
+// about 256 threads below, two elements for the flat box's drop-in forms at
+// p = 3 (15,800 elements, tendency: 0.61 of heve_staged_kernel's time, with four
+// 0.72).
+template <int N1, int MODE, bool FM>
 constexpr int heve_epb() {
-  return N1 == 6 ? 2 : epb_for<N1>();
+  constexpr bool dropin = MODE != MODE_FUSED_GENERAL && MODE != MODE_FUSED_FLAT;
+  return N1 >= 5 ? 1 : N1 == 4 && dropin && FM ? 2 : epb_for<N1>();
+}
+
+// Where heve_staged_kernel runs in place of heve_kernel (which alone holds the
+// filter and the flat box's constants in the drop-in modes).  Measured, this
+// kernel against heve_kernel:
+//  - fused stages at p <= 3: RK4 step at p = 3, 48 x 32 x 10 elements 248 against
+//    313 us (with physics tendencies 318 against 423), at p = 2, 64 x 48 x 12 284
+//    against 330 us; over terrain at p = 3, 62,400 elements 1.50 against 1.94 ms;
+//  - small meshes, at most two workgroups of 256 nodes per CU (one at p = 5): step
+//    over terrain at p = 7, 30 elements 60 against 68 us and 231 elements 79
+//    against 86 us (above it, 488 elements, heve_kernel takes 0.83 of this one's
+//    time), at p = 4, 935 elements 75 against 90 us (2016: 0.80), at p = 5, 72
+//    elements 48 against 49 us (540: 0.90); p = 6 is level at every size;
+//  - drop-in forms with metric arrays, where the difference is smaller: p = 7, 30
+//    elements 22.2 against 23.8 us, p = 3, 62,400 elements HEVE 328 against 347
+//    us (HEVI, whose flux is shorter, 361 against 329 us: heve_kernel).
+enum { STAGED_NEVER = 0, STAGED_SMALL = 1, STAGED_ALWAYS = 2 };
+template <int N1, int MODE>
+constexpr int staged_element_kernel(bool flat) {
+  constexpr bool fused = MODE == MODE_FUSED_GENERAL || MODE == MODE_FUSED_FLAT;
+  constexpr bool cco = MODE == MODE_DROPIN_CCO;
+  if (fused) return N1 <= 4 ? STAGED_ALWAYS : N1 == 7 ? STAGED_NEVER : STAGED_SMALL;
+  if (N1 == 8 && (cco || !flat)) return STAGED_SMALL;
+  if (flat) return STAGED_NEVER;
+  if (N1 == 2) return cco ? STAGED_SMALL : STAGED_ALWAYS;
+  if (N1 == 4) return MODE == MODE_DROPIN_HEVI ? STAGED_NEVER : STAGED_ALWAYS;
+  return N1 == 5 && !cco ? STAGED_SMALL : STAGED_NEVER;
+}
+inline bool small_mesh(const fedg_ctx* ctx) {
+  return (long)ctx->m.Np * ctx->m.Ne <= (ctx->m.n1 == 6 ? 256L : 512L) * ctx->ncu;
 }
 
 template <int MODE>
@@ -1844,21 +2236,36 @@ int launch_heve_mode(fedg_ctx* ctx, const TendIn& in, const RkOut& rk) {
   const DevMesh& m = ctx->m;
   auto go = [&](auto n1c) -> int {
     constexpr int N1 = decltype(n1c)::value;
-    constexpr int EPB = heve_epb<N1>();
-    const dim3 g((m.Ne + EPB - 1) / EPB), b(EPB * N1 * N1 * N1);
+    auto launch = [&](auto kernel, int EPB) {
+      hipLaunchKernelGGL(kernel, dim3((m.Ne + EPB - 1) / EPB), dim3(EPB * N1 * N1 * N1), 0, ctx->stream, m, ctx->c, in,
+                         rk);
+    };
+    constexpr int EPBS = epb_for<N1>();
     if constexpr (MODE == MODE_FUSED_FLAT || MODE == MODE_FUSED_GENERAL) {
       constexpr bool FM = MODE == MODE_FUSED_FLAT;
-      if (in.tp[0] != nullptr)
-        hipLaunchKernelGGL((heve_kernel<N1, EPB, MODE, FM, STAGE_PHYS>), g, b, 0, ctx->stream, m, ctx->c, in, rk);
-      else if (rk.filter)
-        hipLaunchKernelGGL((heve_kernel<N1, EPB, MODE, FM, STAGE_FILTER>), g, b, 0, ctx->stream, m, ctx->c, in, rk);
-      else
-        hipLaunchKernelGGL((heve_kernel<N1, EPB, MODE, FM>), g, b, 0, ctx->stream, m, ctx->c, in, rk);
+      constexpr int EPB = heve_epb<N1, MODE, FM>();
+      constexpr int staged = staged_element_kernel<N1, MODE>(FM);
+      if (rk.filter) {
+        launch(heve_kernel<N1, EPB, MODE, FM, STAGE_FILTER>, EPB);
+      } else if (staged == STAGED_ALWAYS || (staged == STAGED_SMALL && small_mesh(ctx))) {
+        if constexpr (staged != STAGED_NEVER) launch(heve_staged_kernel<N1, EPBS, MODE>, EPBS);
+      } else if constexpr (staged != STAGED_ALWAYS) {
+        if (in.tp[0] != nullptr) launch(heve_kernel<N1, EPB, MODE, FM, STAGE_PHYS>, EPB);
+        else launch(heve_kernel<N1, EPB, MODE, FM>, EPB);
+      }
     } else {
-      if (m.flat)
-        hipLaunchKernelGGL((heve_kernel<N1, EPB, MODE, true>), g, b, 0, ctx->stream, m, ctx->c, in, rk);
-      else
-        hipLaunchKernelGGL((heve_kernel<N1, EPB, MODE, false>), g, b, 0, ctx->stream, m, ctx->c, in, rk);
+      auto form = [&](auto fmc) {
+        constexpr bool FM = decltype(fmc)::value;
+        constexpr int EPB = heve_epb<N1, MODE, FM>();
+        constexpr int staged = staged_element_kernel<N1, MODE>(FM);
+        if (staged == STAGED_ALWAYS || (staged == STAGED_SMALL && small_mesh(ctx))) {
+          if constexpr (staged != STAGED_NEVER) launch(heve_staged_kernel<N1, EPBS, MODE>, EPBS);
+        } else if constexpr (staged != STAGED_ALWAYS) {
+          launch(heve_kernel<N1, EPB, MODE, FM>, EPB);
+        }
+      };
+      if (m.flat) form(std::true_type{});
+      else form(std::false_type{});
     }
     FEDG_HIP_CHECK(hipGetLastError());
     return FEDG_OK;
