@@ -98,27 +98,30 @@ struct fedg_heve {
 
 namespace {
 
-// Horizontally homogeneous base state (every element of a level holds the
-// same values, bit for bit): the flat-box stage kernels read DENS_hyd,
-// PRES_hyd, THERM_hyd, DPhydDx, DPhydDy (host arrays f) from per-level
-// (5, NeZ, Np) tables, which stay in L2, instead of five full fields.
-// *out stays null when the base state varies horizontally.
-int level_tables(const DevMesh& m, const double* const f[5], double** out) {
+// Per-level tables of a horizontally homogeneous base state: DENS_hyd, PRES_hyd,
+// THERM_hyd, DPhydDx, DPhydDy (device fields f) as (5, NeZ, Np) values, which
+// stay in L2, instead of five full fields.  *out stays null when the base state
+// varies horizontally.
+int level_tables(fedg_ctx* ctx, const double* const f[5], double** out) {
   *out = nullptr;
+  const DevMesh& m = ctx->m;
   if (!(m.NeX > 0 && m.NeY > 0 && m.NeZ > 0 && m.Ne == m.NeX * m.NeY * m.NeZ)) return FEDG_OK;
-  const size_t Np = (size_t)m.Np, per = (size_t)m.NeX * m.NeY;
-  bool hom = true;
-  for (int a = 0; a < 5 && hom; ++a)
-    for (size_t ke = 0; ke < (size_t)m.Ne && hom; ++ke) {
-      const size_t rep = (ke / per) * per;
-      hom = memcmp(f[a] + ke * Np, f[a] + rep * Np, Np * sizeof(double)) == 0;
-    }
-  if (!hom) return FEDG_OK;
-  std::vector<double> tab((size_t)5 * m.NeZ * Np);
-  for (int a = 0; a < 5; ++a)
-    for (int kz = 0; kz < m.NeZ; ++kz)
-      memcpy(&tab[((size_t)a * m.NeZ + kz) * Np], f[a] + (size_t)kz * per * Np, Np * sizeof(double));
-  return dev_upload<double>(out, tab.data(), tab.size());
+  const size_t n = (size_t)5 * m.NeZ * m.Np;
+  double* tab = nullptr;  // the tables and, behind them, whether a node differs
+  TRY(dev_upload<double>(&tab, nullptr, n + 1));
+  int differ = 0, rc = FEDG_OK;
+  if (hipMemcpy(tab + n, &differ, sizeof(int), hipMemcpyHostToDevice) != hipSuccess) rc = FEDG_ERR_HIP;
+  if (rc == FEDG_OK) rc = launch_level_tables(ctx, f, tab, reinterpret_cast<int*>(tab + n));
+  if (rc == FEDG_OK && (hipStreamSynchronize(ctx->stream) != hipSuccess ||
+                        hipMemcpy(&differ, tab + n, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess))
+    rc = FEDG_ERR_HIP;
+  if (rc == FEDG_OK && !differ) {
+    *out = tab;
+    return FEDG_OK;
+  }
+  if (rc == FEDG_ERR_HIP) set_error("level tables of the base state: a copy or the kernel failed");
+  (void)hipFree(tab);
+  return rc;
 }
 
 int butcher(const char* name, double dt, fedg_tint* t) {
@@ -1585,10 +1588,10 @@ int fedg_heve_create(fedg_ctx* ctx, const char* scheme, double dt, const double*
       return FEDG_ERR_HIP;
     }
   }
-  // horizontally homogeneous base state: per-level tables for the flat-box stages
-  if (st->flat) {
-    const double* f[5] = {DENS_hyd, PRES_hyd, THERM_hyd, DPhydDx, DPhydDy};
-    rc = level_tables(m, f, &st->lvl);
+  // the kernels of lower orders read the full fields
+  if (st->flat && m.n1 >= 5) {
+    const double* f[5] = {st->DENS_hyd, st->PRES_hyd, st->THERM_hyd, st->DPhydDx, st->DPhydDy};
+    rc = level_tables(ctx, f, &st->lvl);
     if (rc != FEDG_OK) {
       fedg_heve_destroy(st);
       return rc;
@@ -2001,8 +2004,8 @@ int fedg_hevi_create(fedg_ctx* ctx, const char* scheme, double dt, const double*
                    all_equal(CPtot, NpNe, ctx->c.CPdry);
   st->flat7 = m.flat && m.n1 == 8 && m.lift_tensor && dry;
   if (st->flat7) {
-    const double* f[5] = {DENS_hyd, PRES_hyd, THERM_hyd, DPhydDx, DPhydDy};
-    rc = level_tables(m, f, &st->lvl);
+    const double* f[5] = {st->DENS_hyd, st->PRES_hyd, st->THERM_hyd, st->DPhydDx, st->DPhydDy};
+    rc = level_tables(ctx, f, &st->lvl);
     if (rc != FEDG_OK) {
       fedg_hevi_destroy(st);
       return rc;

@@ -117,6 +117,10 @@ struct RkOut {
   int filter;                // FP64 fused, last stage, no physics tendencies: modal filter of the result
 };
 
+// (5, NeZ, Np) tables of the box's five fields from the first element of every
+// level; *differ (zero before) becomes 1 where another element of the level
+// holds other bits
+int launch_level_tables(fedg_ctx* ctx, const double* const f[5], double* tab, int* differ);
 int launch_heve_dropin(fedg_ctx* ctx, const TendIn& in, double* const out[5]);
 int launch_hevi_explicit(fedg_ctx* ctx, const TendIn& in, double* const out[5]);
 // the same tendency on the p = 7 flat-box layout (dry air, in.Rtot null;

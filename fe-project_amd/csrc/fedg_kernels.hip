@@ -2313,6 +2313,26 @@ struct Fields5 {
   double* f[5];
 };
 
+// Every thread compares its node's five values with those of the level's first
+// element, bit for bit; the threads of that element write the table.  One read
+// of the fields (41 x 37 x 13 elements at p = 5, making and freeing a stepper:
+// 29.1 ms with the comparison on the host, 6.6 with this).
+__global__ void level_tables_kernel(const Fields5 f, double* tab, int* differ, int Np, int per, int NeZ, long n) {
+  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n) return;
+  const long ke = t / Np;
+  const int p = (int)(t - ke * Np), kz = (int)(ke / per);
+  const long rep = (long)kz * per * Np + p;
+  bool other = false;
+#pragma unroll
+  for (int v = 0; v < 5; ++v) {
+    const double a = f.f[v][t];
+    other = other | (__double_as_longlong(a) != __double_as_longlong(f.f[v][rep]));
+    if (t == rep) tab[((long)v * NeZ + kz) * Np + p] = a;
+  }
+  if (other) *differ = 1;
+}
+
 // drhot2pres_kernel on the n interior nodes; the threads behind them exchange
 // the halo of the five variables and form DPRES there from the node the
 // exchange copies.  One launch where the parts were seven: launches are what a
@@ -2963,6 +2983,17 @@ int launch_dpres(fedg_ctx* ctx, double* DPRES, const double* DRHOT, const double
   if (n <= 0) return FEDG_OK;
   hipLaunchKernelGGL(dpres_kernel, dim3(nblocks(n, 256)), dim3(256), 0, ctx->stream, DPRES, DRHOT, PRES_hyd,
                      THERM_hyd, Rtot, CVtot, CPtot, n, ctx->c);
+  FEDG_HIP_CHECK(hipGetLastError());
+  return FEDG_OK;
+}
+
+int launch_level_tables(fedg_ctx* ctx, const double* const f[5], double* tab, int* differ) {
+  const DevMesh& m = ctx->m;
+  const long n = (long)m.Np * m.Ne;
+  Fields5 F;
+  for (int v = 0; v < 5; ++v) F.f[v] = const_cast<double*>(f[v]);
+  hipLaunchKernelGGL(level_tables_kernel, dim3(nblocks(n, 256)), dim3(256), 0, ctx->stream, F, tab, differ, m.Np,
+                     m.NeX * m.NeY, m.NeZ, n);
   FEDG_HIP_CHECK(hipGetLastError());
   return FEDG_OK;
 }

@@ -79,3 +79,43 @@ def test_layouts_bitwise(p, NeX, NeY, NeZ, terrain):
             assert np.array_equal(a, b[:n]), f"{name} phys={phys}"
     st.close()
     dm.close()
+
+
+@pytest.mark.parametrize("p", [6, 7])
+def test_base_state_with_one_other_node(p):
+    """A base state that differs from a horizontally homogeneous one by one unit in the last place of one
+    field's last node: the stepper reads that node's own value."""
+    mesh = fedg.BoxMesh(p, 3, 3, 2, (0.0, 3.0e3), (0.0, 3.0e3), (0.0, 1.6e3))
+    c = constants.SCALE
+    nA, n = mesh.Np * mesh.NeA, mesh.Np * mesh.Ne
+    bs0 = cases.base_state(mesh, "constT")
+    bs0 = dataclasses.replace(bs0, Rtot=np.full(nA, c.Rdry), CVtot=np.full(nA, c.CVdry), CPtot=np.full(nA, c.CPdry))
+    om = O.OracleMesh(mesh)
+    dm = fedg.DeviceMesh(mesh)
+    rng = np.random.default_rng(p)
+    q = [mesh.field() for _ in range(5)]
+    for f, amp in zip(q, (1e-3, 0.3, 0.5, 5.0, 1.0)):
+        f[:n] = amp * rng.standard_normal(n)
+        om.exchange(f)
+    for field in ("DENS_hyd", "PRES_hyd", "THERM_hyd", "DPhydDx", "DPhydDy", None):
+        print(f"base state with one other node, p={p} {field}", flush=True)
+        bs = bs0
+        Dx, Dy = om.calc_phyd_hgrad(bs)
+        if field in ("DPhydDx", "DPhydDy"):
+            f = Dx if field == "DPhydDx" else Dy
+            f[n - 1] += 1.0e-3
+        elif field:
+            f = getattr(bs, field).copy()
+            f[n - 1] = np.nextafter(f[n - 1], np.inf)
+            om.exchange(f)
+            bs = dataclasses.replace(bs, **{field: f})
+        st = fedg.HeveStepper(dm, bs, Dx, Dy, 0.01)
+        st.set_state(q)
+        st.run(1)
+        g = st.get_state()
+        st.close()
+        r = [a.copy() for a in q]
+        om.heve_update(r, bs, Dx, Dy, 0.01, 1)
+        for name, a, b in zip(fedg.VARS, g, r):
+            assert np.array_equal(a, b[:n]), f"{name} {field}"
+    dm.close()
