@@ -408,10 +408,28 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// exchanges two register pairs where they are
+// exchanges two register pairs where they are: through a third, or (HALVES)
+// half by half without one, which is slower but lets the n = 24 solve with row
+// exchanges spill 24 registers where it spills 55
+template <bool HALVES>
 __device__ __forceinline__ void swap_in_place(double& x, double& y) {
-  double t;
-  asm("v_mov_b64 %2, %0\n\tv_mov_b64 %0, %1\n\tv_mov_b64 %1, %2" : "+v"(x), "+v"(y), "=&v"(t));
+  if constexpr (HALVES) {
+    int x0 = __double2loint(x), x1 = __double2hiint(x), y0 = __double2loint(y), y1 = __double2hiint(y);
+    asm("v_swap_b32 %0, %1" : "+v"(x0), "+v"(y0));
+    asm("v_swap_b32 %0, %1" : "+v"(x1), "+v"(y1));
+    x = __hiloint2double(x1, x0);
+    y = __hiloint2double(y1, y0);
+  } else {
+    double t;
+    asm("v_mov_b64 %2, %0\n\tv_mov_b64 %0, %1\n\tv_mov_b64 %1, %2" : "+v"(x), "+v"(y), "=&v"(t));
+  }
+}
+
+// max(|a|, |b|); a NaN is passed over unless both are
+__device__ __forceinline__ double max_abs(double a, double b) {
+  double r;
+  asm("v_max_f64 %0, |%1|, |%2|" : "=v"(r) : "v"(a), "v"(b));
+  return r;
 }
 
 // row i of the block is complete here (no instruction)
@@ -425,9 +443,9 @@ __device__ __forceinline__ void keep_order(double (&A)[NS][n], double (&B)[n], i
 // then back substitution: B becomes the solution (lanes 0..3).
 // PIVOT false: no rows are exchanged; false is returned when a line's pivot
 // was not on the diagonal (its result is then to be discarded), so that the
-// usual path is one stretch of code without a branch, whose registers hold
-// the blocks.  PIVOT true: rows are exchanged in the registers (the branches
-// make the allocator spill).
+// path is one stretch of code without a branch, whose registers hold the
+// blocks.  PIVOT true: rows are exchanged in the registers (the branches make
+// the allocator spill at n >= 21).
 // ahead() is called in the back substitution once registers have come free:
 // the next level's loads, whose latency the rest of it covers.
 template <int NS, int N, int SEG, bool PIVOT, class F>
@@ -438,9 +456,18 @@ __device__ __forceinline__ bool lu_solve_cols(double (&A)[NS][NS * N], double (&
   static_for<0, n>([&](auto K) __attribute__((always_inline)) {
     constexpr int k = decltype(K)::value, ck = k / NS, sk = k % NS;
     if constexpr (k < n - 1) {
-      bool larger = false;
+      // the largest entry below the diagonal, by halves: one chain of five
+      // instead of a compare and a mask per entry
+      constexpr int m = n - 1 - k;
+      double top[m];
 #pragma unroll
-      for (int i = k + 1; i < n; ++i) larger = larger | (fabs(A[sk][i]) > fabs(A[sk][k]));
+      for (int i = 0; i < m; ++i) top[i] = A[sk][k + 1 + i];
+#pragma unroll
+      for (int d = 1; d < m; d *= 2)
+#pragma unroll
+        for (int i = 0; i + d < m; i += 2 * d) top[i] = max_abs(top[i], top[i + d]);
+      const double big = fabs(top[0]);
+      const bool larger = big > fabs(A[sk][k]);
       const unsigned long long here = __ballot(larger & (c == ck));
       if constexpr (!PIVOT) {
         off |= here;
@@ -449,9 +476,6 @@ __device__ __forceinline__ bool lu_solve_cols(double (&A)[NS][NS * N], double (&
         // the first largest entry of a column with a larger one (NaN entries
         // are passed over, a NaN on the diagonal stays, as in the reference's
         // running comparison)
-        double big = fabs(A[sk][k]);
-#pragma unroll
-        for (int i = k + 1; i < n; ++i) big = __builtin_fmax(big, fabs(A[sk][i]));
         int p = k;
 #pragma unroll
         for (int i = n - 1; i > k; --i) p = fabs(A[sk][i]) == big ? i : p;
@@ -461,8 +485,8 @@ __device__ __forceinline__ bool lu_solve_cols(double (&A)[NS][NS * N], double (&
         for (int i = k + 1; i < n; ++i) {
           if (p == i) {
 #pragma unroll
-            for (int s = 0; s < NS; ++s) swap_in_place(A[s][i], A[s][k]);
-            swap_in_place(B[i], B[k]);
+            for (int s = 0; s < NS; ++s) swap_in_place<(n > 21)>(A[s][i], A[s][k]);
+            swap_in_place<(n > 21)>(B[i], B[k]);
           }
         }
         inv = 1.0 / A[sk][k];
@@ -723,10 +747,21 @@ __global__ void __launch_bounds__(64 * LineSeg<N1>::WPB) hevi_solve_uv_kernel(co
 // right-hand side and the coupling to the level above, and passes them
 // through LDS to the lanes that hold those columns; every lane forms the
 // other columns of its own node from the rows' metric factors.
-// MODE: SOLVE_ALL, every line with row exchanges (p <= 3, whose blocks leave
-// room for them); at p >= 4 SOLVE_DIAGONAL, which gives the groups of lines
-// whose pivots leave the diagonal up to the list a.flagged (count, then group
-// numbers), and SOLVE_FLAGGED, which solves those.
+// MODE: SOLVE_ALL, every line with row exchanges; SOLVE_DIAGONAL, which gives
+// the groups of lines whose pivots leave the diagonal up to the list a.flagged
+// (count, then group numbers), and SOLVE_FLAGGED, which solves those.  The
+// exchanges' branches make the allocator spill at p = 6 (5 registers) and p = 7
+// (24), none below.  Drop-in stage, pivots on the diagonal / off it in every
+// block, SOLVE_ALL against the other two:
+//   p = 5, 64 x 32 x 8 elements 1066 / 1260 against 1055 / 1366 us; 8 x 4 x 4
+//   85 / 99 against 86 / 114 us;
+//   p = 6, 64 x 32 x 8 1799 / 2058 against 1766 / 2270 us; 8 x 4 x 4 101 / 121
+//   against 99 / 139 us;
+//   p = 7, 64 x 32 x 8 2552 / 2980 against 2413 / 3306 us; 16 x 8 x 8 (a group per
+//   SIMD) 287 / 346 against 284 / 378 us; 8 x 4 x 4 113 / 140 against 112 / 166 us.
+// So SOLVE_ALL below p = 7, and there on meshes of no more groups than SIMDs,
+// where the spills hide behind the latency; beyond, the usual steps, whose
+// pivots stay on the diagonal, decide.
 enum { SOLVE_ALL = 0, SOLVE_DIAGONAL = 1, SOLVE_FLAGGED = 2 };
 template <int N1>
 struct LineLds {
@@ -1325,9 +1360,9 @@ int run_newton(fedg_ctx* ctx, HeviArgs& a, HeviWork* w, int max_it, double rtol,
       if (rtol > 0.0 && it > 0 && r > 0.5 * r_prev) break;
       r_prev = r;
     }
-    if constexpr (N1 <= 4) {
+    if (N1 <= 7 || ngroup <= (long)4 * ctx->ncu) {
       hipLaunchKernelGGL((hevi_solve3_kernel<N1, SOLVE_ALL>), gline, bline, 0, ctx->stream, a);
-    } else {
+    } else if constexpr (N1 > 7) {
       hipLaunchKernelGGL((hevi_solve3_kernel<N1, SOLVE_DIAGONAL>), gline, bline, 0, ctx->stream, a);
       FEDG_HIP_CHECK(hipGetLastError());
       hipLaunchKernelGGL((hevi_solve3_kernel<N1, SOLVE_FLAGGED>), gflag, bline, 0, ctx->stream, a);

@@ -251,6 +251,8 @@ int oracle_hevi_newton(const oracle_mesh *m, double *const pv[5], const double *
                        const double *const q0[5], const double *DENS_hyd, const double *PRES_hyd,
                        const double *Rtot, const double *CVtot, const double *CPtot, double impl_fac, double dt,
                        int max_it, double rtol, double *resid);
+/* marks in lines (Nfp, Ne2D) the columns in which the three-variable solves that follow exchange rows; null: stop */
+void oracle_hevi_mark_pivots(unsigned char *lines);
 /* r0_ext > 0: the residual norm the tolerance is relative to */
 int oracle_hevi_newton_r0(const oracle_mesh *m, double *const pv[5], const double *const qs[5],
                           const double *const q0[5], const double *DENS_hyd, const double *PRES_hyd,

@@ -7,6 +7,7 @@ restates the reference Fortran on the CPU.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes as C
 import os
 
@@ -85,6 +86,8 @@ def _load():
                                                                         C.c_double, C.c_double, dp]
     lib.oracle_hevi_newton_r0.restype = C.c_int
     lib.oracle_modalfilter_apply.argtypes = [M] + [dp] * 5 + [C.c_int]
+    lib.oracle_hevi_mark_pivots.argtypes = [C.c_void_p]
+    lib.oracle_hevi_mark_pivots.restype = None
     lib.oracle_hevi_cal_vi.argtypes = [M, V5, V5, V5] + [dp] * 5 + [C.c_double, C.c_double, C.c_int,
                                                                      C.c_double, dp]
     lib.oracle_hevi_cal_vi.restype = C.c_int
@@ -362,6 +365,18 @@ class OracleMesh:
 
     def _v5(self, fields):
         return (dp * 5)(*[_d(a) for a in fields])
+
+    @contextlib.contextmanager
+    def pivot_lines(self):
+        """Flags (Nfp, Ne2D in memory order) of the vertical lines whose three-variable solves exchange rows inside
+        the block."""
+        m = self.mesh
+        flags = np.zeros(m.Ne2D * (m.porder + 1) ** 2, dtype=np.uint8)
+        LIB.oracle_hevi_mark_pivots(flags.ctypes.data_as(C.c_void_p))
+        try:
+            yield flags
+        finally:
+            LIB.oracle_hevi_mark_pivots(None)
 
     def hevi_cal_vi(self, q, var0, bs, impl_fac, dt, max_it=1, rtol=0.0):
         """Implicit tendencies in VID order (each (Np,NeA)), iterations done, residual history."""

@@ -580,9 +580,10 @@ static void hevi_matbnd_uv(const hevi_ctx *h, int ke2D, int ij, int kz, double *
 /* solve_Nnode8_var3 / solve_Nnode8_uv (..._linalgebra.F90:2142-2445), one
  * column: LU with partial pivoting of the n x n block A (column-major,
  * overwritten), then nr right-hand sides X (n x nr, column-major).  When
- * is_top is false, the rhs are b followed by the columns of G. */
-static void hevi_lu_solve(int n, double *A, int nr, double *X) {
-  int ipiv[64];
+ * is_top is false, the rhs are b followed by the columns of G.  Returns the
+ * number of row exchanges. */
+static int hevi_lu_solve(int n, double *A, int nr, double *X) {
+  int ipiv[64], exchanges = 0;
   for (int k = 0; k < n; ++k) {
     double tmpv = fabs(A[k + n * k]);
     ipiv[k] = k;
@@ -594,6 +595,7 @@ static void hevi_lu_solve(int n, double *A, int nr, double *X) {
       }
     }
     const int ip = ipiv[k];
+    if (ip != k) ++exchanges;
     if (ip != k)
       for (int j = 0; j < n; ++j) {
         const double t = A[k + n * j];
@@ -627,7 +629,13 @@ static void hevi_lu_solve(int n, double *A, int nr, double *X) {
       for (int j = i + 1; j < n; ++j) t = t - A[i + n * j] * X[j + n * r];
       X[i + n * r] = t * A[i + n * i];
     }
+  return exchanges;
 }
+
+/* test instrumentation: lines (Nfp, Ne2D) of the three-variable solve in which
+ * rows were exchanged are marked here until it is set to null */
+static unsigned char *pivot_lines = 0;
+void oracle_hevi_mark_pivots(unsigned char *lines) { pivot_lines = lines; }
 
 /* solve_uv (..._common_2.F90:589-689): block Thomas over the column, then
  * MOMX, MOMY += increment */
@@ -659,7 +667,7 @@ static void hevi_solve_uv(hevi_ctx *h) {
               Xk[pv + N] = Xk[pv + N] - tmp * Xp[(N - 1) + N];
             }
           }
-          hevi_lu_solve(N, D, kz == NeZ - 1 ? 2 : 3, Xk);
+          (void)hevi_lu_solve(N, D, kz == NeZ - 1 ? 2 : 3, Xk);
         }
         for (int kz = NeZ - 2; kz >= 0; --kz) {
           double *Xk = X + (long)N * 3 * kz;
@@ -714,7 +722,7 @@ static void hevi_solve_var3(hevi_ctx *h) {
               Xk[r] = Xk[r] - t1 * Xp[p1] - t2 * Xp[p2] - t3 * Xp[p3];
             }
           }
-          hevi_lu_solve(n3, D, kz == NeZ - 1 ? 1 : 4, Xk);
+          if (hevi_lu_solve(n3, D, kz == NeZ - 1 ? 1 : 4, Xk) && pivot_lines) pivot_lines[ke2D * Nfp + ij] = 1;
         }
         for (int kz = NeZ - 2; kz >= 0; --kz) {
           double *Xk = X + (long)n3 * 4 * kz;
