@@ -489,7 +489,9 @@ static int mlp_sync_weights(MlpImpl* p) {
 // SIMD two; below, four times as many wavefronts of 16 x 16 hide the latency.
 // Forward, 641-256-256-256-320, wide / narrow: 2048 rows (512 wide tiles in a
 // hidden layer) 47.8 / 37.8 us, 4096 rows 52.6 / 50.2, 8192 rows (2048 tiles)
-// 67.1 / 71.9, 65536 rows 363 / 413 us.
+// 67.1 / 71.9, 65536 rows 363 / 413 us.  Loss and gradients, the backward pass
+// wide / narrow: 2048 rows 85 / 84 us, 4096 rows 125 / 128, 8192 rows 199 / 205,
+// 65536 rows 1907 / 1934 us; 1024-wide layers, 8192 rows 889 / 936 us.
 static bool wide_tiles(int M, int N) { return (long)(pad32(M) / 32) * (pad32(N) / 32) >= 2048; }
 
 // forward of B rows of X (device fp32 [B x n_in]) into Y; train: what the backward pass reads as well
@@ -526,7 +528,7 @@ static int mlp_bwd(MlpImpl* p, int B) {
     a.nW = tile_blocks<1>(a.N, a.K);
     a.nX = a.nW + (a.N + 15) / 16;
     unsigned blocks = a.nX;
-    const bool wide = wide_tiles(B, a.K);
+    const bool wide = l > 0 && wide_tiles(B, a.K);  // of the input gradient, which the first layer has none of
     if (l > 0) {
       a.H = p->act[l];
       a.dX32 = p->dact[l];
