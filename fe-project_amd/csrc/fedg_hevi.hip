@@ -1259,17 +1259,11 @@ void launch_rhs3(fedg_ctx* ctx, const HeviArgs& a) {
     hipLaunchKernelGGL((hevi_rhs3_kernel<N1, false>), dim3(m.Ne), dim3(N1 * N1 * N1), 0, ctx->stream, a);
 }
 
-// Columns taken: those whose levels' solutions fit a 64 KB block of one
-// wavefront in the row-per-lane layout (64 / seg lines of n (n + 1) / 2 + seg
-// entries of U, 4 n per level and 13 N1 coefficients).
-template <int N1>
-bool column_fits(int NeZ) {
-  constexpr int n3 = 3 * N1;
-  constexpr int seg3 = n3 <= 8 ? 8 : (n3 <= 16 ? 16 : 32), segu = N1 <= 8 ? 8 : 16;
-  const size_t l3 = 2 * N1 * N1 + (size_t)(64 / seg3) * (13 * N1 + n3 * (n3 + 1) / 2 + seg3 + (size_t)NeZ * 4 * n3);
-  const size_t lu = (size_t)(64 / segu) * (N1 * (N1 + 1) / 2 + segu + (size_t)NeZ * 3 * N1);
-  return sizeof(double) * l3 <= 64 * 1024 && sizeof(double) * lu <= 64 * 1024;
-}
+// Tallest column taken, in elements, by N1.  The kernels set no limit of their
+// own (a wavefront's scratch grows with NeZ); these are the limits the entry
+// points have always had, and what the no-allocation entry's fixed scratch is
+// sized for.
+constexpr int kMaxNeZ[9] = {0, 0, 40, 53, 39, 30, 52, 43, 37};
 
 // finish: what the solve of DENS, MOMZ and RHOT of the last iteration stores,
 // where that iteration is known beforehand (no tolerance, no residual asked
@@ -1280,7 +1274,7 @@ int run_newton(fedg_ctx* ctx, HeviArgs& a, HeviWork* w, int max_it, double rtol,
   const DevMesh& m = ctx->m;
   double* const partial = w->partial;
   double* const partial_h = w->partial_h;
-  if (!column_fits<N1>(a.NeZ)) {
+  if (a.NeZ > kMaxNeZ[N1]) {
     set_error("HEVI: too many elements in the vertical for the line solve (NeZ)");
     return FEDG_ERR_UNSUPPORTED;
   }
@@ -1634,8 +1628,8 @@ static __device__ __align__(256) double scratch[kScratchDoubles];
 
 // The line solves' scratch of the same calls, apart from it so that the
 // meshes the workspace takes do not change: 32 MiB hold the level solutions
-// of 682 wavefronts at p = 7 and NeZ = 8, and of at least 147 for every
-// column accepted (the wavefronts in flight walk the lines).
+// of 682 wavefronts at p = 7 and NeZ = 8, and of at least 136 for every mesh
+// taken (p = 2 at 53 levels; the wavefronts in flight walk the lines).
 constexpr size_t kLineScratchDoubles = (size_t)4 << 20;
 
 static __device__ __align__(256) double line_scratch[kLineScratchDoubles];

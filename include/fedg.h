@@ -423,7 +423,11 @@ int fedg_hevi_cal_tend(fedg_ctx *ctx, double *DENS_dt, double *MOMX_dt, double *
  * abstract interface atm_dyn_nonhydro3d_cal_vi
  * (FDS/scale_atm_dyn_dgm_driver_nonhydro3d.F90:201-250) minus the derived
  * types; fields (Np,NeA) on the device; the mesh must be one box column
- * stack (elements numbered horizontally first). */
+ * stack (elements numbered horizontally first).  impl_fac != 0 takes at most
+ * 40, 53, 39, 30, 52, 43, 37 elements in the vertical for p = 1 .. 7, here and
+ * in every implicit solve below (else FEDG_ERR_UNSUPPORTED).  The first call on
+ * a context allocates its workspace: 13 Np Ne + 2 Nfp Ne doubles and, for the
+ * line solves, 12 Np Ne more but no more than 1 GB. */
 int fedg_hevi_cal_vi(fedg_ctx *ctx, double *DENS_dt, double *MOMX_dt, double *MOMY_dt, double *MOMZ_dt,
                      double *RHOT_dt, const double *DDENS_, const double *MOMX_, const double *MOMY_,
                      const double *MOMZ_, const double *DRHOT_, const double *DENS_hyd,
@@ -451,8 +455,8 @@ int fedg_hevi_cal_vi_newton(fedg_ctx *ctx, double *DENS_dt, double *MOMX_dt, dou
  * same results bit for bit) for callers that cannot allocate device memory
  * (code under HIP graph capture, tight serving loops, hosts that forbid
  * hipMalloc).  Its implicit-solve workspace is a fixed 64 MiB device array of
- * the library instead of a hipMalloc'd one; the call allocates and frees
- * nothing.  Meshes whose workspace (13 Np Ne + 2 Nfp Ne doubles, each part
+ * the library (and one of 32 MiB for the line solves, which sets no limit)
+ * instead of a hipMalloc'd one; the call allocates and frees nothing.  Meshes whose workspace (13 Np Ne + 2 Nfp Ne doubles, each part
  * rounded to 256 B, plus 2 KiB) exceeds 64 MiB are rejected with
  * FEDG_ERR_UNSUPPORTED (at p = 7 about 1200 elements).  Every call on one
  * device shares the workspace: calls that overlap in time on the same device

@@ -58,12 +58,12 @@ def test_line_solves_bitwise(p, NeX, NeY, NeZ, impl_fac):
     dm.close()
 
 
-def mixed_state(m, seed, amp=1.0):
+def mixed_state(m, seed):
     rng = np.random.default_rng(seed)
     n = m.Np * m.Ne
     q = [m.field() for _ in range(5)]
     for f, a in zip(q, (1e-3, 0.3, 0.5, 5.0, 1.0)):
-        f[:n] = amp * a * rng.standard_normal(n)
+        f[:n] = a * rng.standard_normal(n)
         m.exchange(f)
     return q
 
@@ -102,3 +102,37 @@ def test_mixed_pivots_and_many_groups(p, NeX, NeY, NeZ, impl_fac, noalloc, excha
     for name, a, b in zip(fedg.VARS, [g[0], g[4], g[3], g[1], g[2]], ref):
         assert np.array_equal(a[:n], b[:n], equal_nan=True), name
     dm.close()
+
+
+# the tallest column of every order
+TALLEST = {1: 40, 2: 53, 3: 39, 4: 30, 5: 52, 6: 43, 7: 37}
+
+
+@pytest.mark.parametrize("p", range(1, 8))
+def test_tallest_column(p):
+    print(f"line solves, tallest column p={p}", flush=True)
+    for NeZ in (TALLEST[p], TALLEST[p] + 1):
+        m = fedg.BoxMesh(p, 2, 1, NeZ, (0.0, 2.0e3), (0.0, 1.0e3), (0.0, 2.5e2 * NeZ))
+        bs = cases.base_state(m, "constBVFreq")
+        om = O.OracleMesh(m)
+        dm = fedg.DeviceMesh(m)
+        n = m.Np * m.Ne
+        q, q0 = mixed_state(m, p), mixed_state(m, p + 100)
+        dev = lambda a: fedg.DevField(a.size, a)  # noqa: E731
+        d, d0 = [dev(a) for a in q], [dev(a) for a in q0]
+        aux = [dev(getattr(bs, k)) for k in ("DENS_hyd", "PRES_hyd", "Rtot", "CVtot", "CPtot")]
+        for noalloc in (False, True):
+            out = [dev(m.field()) for _ in range(5)]
+            call = lambda: fedg.hevi_cal_vi(dm, out, d[0], d[3], d[4], d[2], d[1], aux[0], aux[1], d0[0], d0[3],  # noqa: E731
+                                            d0[4], d0[2], d0[1], *aux[2:], 0.02, 1.0,
+                                            **(dict(max_it=1, noalloc=True) if noalloc else {}))
+            if NeZ > TALLEST[p]:
+                with pytest.raises(fedg.FedgError, match="too many elements in the vertical"):
+                    call()
+                continue
+            call()
+            ref, _, _ = om.hevi_cal_vi(q, q0, bs, 0.02, 1.0)
+            g = [a.download() for a in out]
+            for name, a, b in zip(fedg.VARS, [g[0], g[4], g[3], g[1], g[2]], ref):
+                assert np.array_equal(a[:n], b[:n], equal_nan=True), f"{name} noalloc={noalloc}"
+        dm.close()
