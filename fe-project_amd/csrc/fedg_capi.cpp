@@ -1240,8 +1240,9 @@ int hevi_work_get(fedg_ctx* ctx, HeviWork** w) {
     rc = FEDG_ERR_NOMEM;
   }
   h->partial_h = h->partial;
-  // line-solve scratch: 16 wavefronts per CU (twice what is resident at p = 7,
-  // so that the last ones balance), no more than the lines fill
+  // Line-solve scratch: 16 wavefronts per CU (twice what is resident at p = 7,
+  // so that the last ones balance), no more than the lines fill: 12 doubles per
+  // node up to that, and at most 201 MB at p = 7 with 8 levels, 931 MB with 37
   const size_t lpw = m.n1 <= 4 ? 16 : 8, nline = (size_t)m.Ne2D * m.Nfp;
   const size_t nwave = std::min(((nline + lpw - 1) / lpw + 1) / 2 * 2, (size_t)16 * ctx->ncu);
   h->lines_n = line_list_doubles((long)((nline + lpw - 1) / lpw)) + nwave * line_scratch_per_wave(m.n1, m.Ne / m.Ne2D);
@@ -1754,7 +1755,13 @@ static int heve_step(fedg_heve* st, std::vector<hipEvent_t>* evs, size_t* ev_i) 
   const int q0 = st->q0;
   int cur = q0;
   int last_out = q0;
-  // the filter joins the last stage's kernel, except in FP32 and with physics tendencies
+  // The filter joins the last stage's kernel, except in FP32 and with physics
+  // tendencies.  At p = 7 on the flat box that stage then runs in the general
+  // kernel instead of the p = 7 one, and is still the faster way: step fused /
+  // with the filter's own launches, p = 7 flat, 480 elements 88 / 94 us, 7920
+  // elements 990 / 1031 us; p = 5 flat, 18330 elements 1141 / 1242 us; p = 3 over
+  // terrain, 62400 elements 1598 / 1613 us (0.87 to 0.99 over every order, size
+  // and both metrics)
   const bool fuse_filter = st->mfilter && !st->fp32 && !st->tp[0];
   for (int s = 1; s <= t.nstage; ++s) {
     RkOut rk{};

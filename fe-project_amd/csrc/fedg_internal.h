@@ -208,8 +208,9 @@ int launch_drhot2pres(fedg_ctx* ctx, double* PRES, double* DPRES, const double* 
                       const double* PRES_hyd, const double* THERM_hyd, const double* Rtot,
                       const double* CVtot, const double* CPtot, long n);
 int launch_halo_exchange(fedg_ctx* ctx, double* const* fields, int nfields);
-// DPRES (and PRES unless null) of the state q with both halos: the exchange of
-// the five variables, DRHOT2PRES and the exchange of DPRES
+// The exchange of the five variables of the state q, DRHOT2PRES (DPRES and,
+// unless null, PRES) and the exchange of DPRES in one launch; PRES is written on
+// the interior nodes only
 int launch_pressure_halo(fedg_ctx* ctx, double* const q[5], double* PRES, double* DPRES, const double* PRES_hyd,
                          const double* THERM_hyd, const double* Rtot, const double* CVtot, const double* CPtot);
 int launch_apply_bc(fedg_ctx* ctx, double* MOMX, double* MOMY, double* MOMZ);

@@ -1992,8 +1992,9 @@ __global__ void __launch_bounds__(256) diagvar_kernel(const DiagVar a, const Con
 // Bound: the ordered sums' chains, then HBM traffic.  No species' sums depend on
 // another's correction, so all of them are formed at once, a lane each: two
 // chains per element where there were nq + 1.  NQ: room for species; four keep
-// the sums' terms at 33 KB per element of p = 7.  32 x 32 x 16 elements, three
-// species: 895 -> 371 us.
+// the sums' terms at 33 KB per element of p = 7, where 64 VGPRs (two of them
+// spilled) then let four elements on a CU.  32 x 32 x 16 elements, three species:
+// 895 -> 371 us.
 template <int N1, int EPB, int NQ>
 __global__ void __launch_bounds__(EPB * N1 * N1 * N1) __attribute__((amdgpu_waves_per_eu(NQ == 4 && N1 == 8 ? 8 : 4)))
 negfix_kernel(const DevMesh m, const Consts c, const NegFix a) {
