@@ -1,13 +1,17 @@
-"""CPU check of the indices the flat-box stage kernels form by arithmetic
+"""CPU check of the indices the flat-box element kernels form by arithmetic
 instead of loading vmapM / vmapP: the element each thread of each workgroup
-works on (xcd_remap, several elements per workgroup, padding elements in the
-last workgroup) and the exterior node of every face node (neighbour element
-and its opposite face node, or the own node at a closed boundary).
+works on (xcd_remap or the block number itself, several elements per workgroup,
+padding elements in the last workgroup), the exterior node of every face node
+(neighbour element and its opposite face node, or the own node at a closed
+boundary), and the places in the per-level base-state tables.
 
-The same arithmetic as heve_kernel<N1, EPB, MODE_FUSED_FLAT> and heve7_body
+The same arithmetic as heve_kernel and heve_staged_kernel in MODE_FUSED_FLAT,
+their drop-in forms' element mapping and own face nodes, and heve7_body
 (fe-project_amd/csrc/fedg_kernels.hip, fedg_device.h), restated here and
 compared with the builder's maps, which the general kernels load:
-  - every element below Ne is taken by exactly one (workgroup, slot);
+  - every element below Ne is taken by exactly one (workgroup, slot), with the
+    elements per workgroup of heve_kernel's fused and drop-in forms (heve_epb),
+    of heve_staged_kernel (epb_for) and of heve7;
   - padding slots (ke >= Ne) exist only in the workgroup that xcd_remap sends
     to the last block, and the kernels load nothing for them;
   - an open face's exterior node is vmapP - 1, resolved through the halo slot
@@ -15,7 +19,11 @@ compared with the builder's maps, which the general kernels load:
     vmapM - 1, which the halo slot vmapP points to copies, with the boundary's
     velocity BC;
   - every index formed for a valid element is below Np * Ne (the fused
-    stepper's fields have no halo tail).
+    stepper's fields have no halo tail), and the drop-in forms' vmapP below
+    Np * NeA;
+  - the table places of the own node, of a face's own side and of its exterior
+    side (oh, hM, hP) lie in the (NeZ, Np) table and belong to the level and
+    node of the element they stand for.
 Meshes cover p = 1..7, a number of elements that is and is not a multiple of
 the elements per workgroup and of 8, and periodic and walled boundaries,
 including the 5 x 3 x 4 p = 1 box of a removed tracer-kernel variant that once
@@ -45,7 +53,7 @@ def face_node(N1, f, a):
 
 
 def exterior(mesh, ke, f, a):
-    """Exterior node of face node a of face f of element ke, as the flat kernels form it."""
+    """Exterior side of face node a of face f of element ke, as flat_exterior forms it: index, closed, table place."""
     N1, Np = mesh.porder + 1, mesh.Np
     NeX, NeY, NeZ = mesh.NeX, mesh.NeY, mesh.NeZ
     px, py, pz = mesh.periodic
@@ -76,15 +84,21 @@ def exterior(mesh, ke, f, a):
         nk += 1
         if nk >= NeZ:
             nk, closed = (0, False) if pz else (nk, True)
+    node = face_node(N1, f if closed else OPP[f], a)
     if closed:
-        return Np * ke + face_node(N1, f, a), True
-    return Np * (ni + NeX * (nj + NeY * nk)) + face_node(N1, OPP[f], a), False
+        ni, nj, nk = ei, ej, ek
+    return Np * (ni + NeX * (nj + NeY * nk)) + node, closed, Np * nk + node
 
 
 def epb_for(N1):
-    """Elements per workgroup of heve_kernel (fedg_kernels.hip epb_for)."""
+    """Elements per workgroup of heve_staged_kernel (fedg_kernels.hip epb_for)."""
     Np = N1 ** 3
     return 1 if Np >= 128 else 256 // Np
+
+
+def heve_epb(N1, dropin):
+    """Elements per workgroup of heve_kernel on the flat box (fedg_kernels.hip heve_epb)."""
+    return 1 if N1 >= 5 else 2 if N1 == 4 and dropin else epb_for(N1)
 
 
 MESHES = [
@@ -111,16 +125,17 @@ def test_flat_kernel_indices_match_builder_maps(p, NeX, NeY, NeZ, periodic):
     velbc = mesh.velbc([0 if periodic[a] else BND_SLIP for a in (1, 0, 1, 0, 2, 2)])
     vmapM = mesh.vmapM.reshape(Ne, NfpTot) - 1
     vmapP = mesh.vmapP.reshape(Ne, NfpTot) - 1
-    # heve_kernel<N1, EPB, MODE_FUSED_FLAT>: nblk workgroups of EPB elements,
-    # and the p = 7 heve7 kernels: Ne workgroups of one element
-    layouts = [(epb_for(N1), -(-Ne // epb_for(N1)))]
+    # workgroups of EPB elements, in xcd_remap's order or (the staged kernel's
+    # drop-in forms) their own
+    layouts = {(heve_epb(N1, False), True), (heve_epb(N1, True), True), (epb_for(N1), True), (epb_for(N1), False)}
     if N1 == 8:
-        layouts.append((1, Ne))
-    for EPB, nblk in layouts:
+        layouts.add((1, True))  # heve7
+    for EPB, remapped in sorted(layouts):
+        nblk = -(-Ne // EPB)
         taken = np.zeros(Ne, dtype=np.int64)
         padding_blocks = set()
         for b in range(nblk):
-            blk = xcd_remap(b, nblk)
+            blk = xcd_remap(b, nblk) if remapped else b
             assert 0 <= blk < nblk
             for e in range(EPB):
                 ke = blk * EPB + e
@@ -132,14 +147,22 @@ def test_flat_kernel_indices_match_builder_maps(p, NeX, NeY, NeZ, periodic):
         assert padding_blocks <= {nblk - 1}, "padding only in the last block"
         assert nblk * EPB - Ne < EPB
     # exterior node of every face node of every element
+    per, table = NeX * NeY, Np * NeZ
     for ke in range(Ne):
+        ek = ke // per
+        assert 0 <= Np * ek and Np * ek + Np - 1 < table  # oh of the element's nodes
         for f in range(6):
             for a in range(Nfp):
                 fp = f * Nfp + a
                 iM = Np * ke + face_node(N1, f, a)
                 assert iM == vmapM[ke, fp]
-                iP, closed = exterior(mesh, ke, f, a)
+                iP, closed, hP = exterior(mesh, ke, f, a)
                 assert 0 <= iP < Np * Ne
+                assert 0 <= vmapP[ke, fp] < Np * mesh.NeA
+                hM = Np * ek + face_node(N1, f, a)
+                assert 0 <= hM < table and 0 <= hP < table
+                assert hM == Np * (iM // Np // per) + iM % Np
+                assert hP == Np * (iP // Np // per) + iP % Np
                 # vmapP points into the halo tail at the domain boundary (the
                 # single-tile exchange fills the slot from halo_src)
                 slot = vmapP[ke, fp] - Np * Ne
