@@ -330,9 +330,9 @@ __device__ __forceinline__ void hevi_rhs3_body(const HeviArgs& a) {
 //    sides of every line of the wavefront;
 //  - rows are exchanged in the registers, only when a line's pivot is not on
 //    the diagonal (rare for the diagonally dominant blocks of the usual steps).
-// Bound: FP64 VALU issue (about 5,700 instructions per level of eight p = 7
+// Bound: FP64 VALU issue (about 5,500 instructions per level of eight p = 7
 // lines, 11 per multiplier: product, two moves, four multiply-subtract pairs;
-// VALU busy 0.78 of the time).  A block needs 2 n (NS + 1) VGPRs (192 at
+// VALU busy 0.84 of the time).  A block needs 2 n (NS + 1) VGPRs (192 at
 // p = 7), so two wavefronts share a SIMD and nothing else may stay in
 // registers across the LU: a spilled address waits, in the one order vector
 // memory completes in, for the stores before it (with 40 spilled registers

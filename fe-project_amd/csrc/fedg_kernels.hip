@@ -982,7 +982,7 @@ __device__ __forceinline__ void rusanov32_hevi(const Side32& M, const Side32& P,
 //    in flight before the first barrier.
 // Measured (64 x 64 x 16 elements, RK4 step): every sum formed on the spot
 // (124 -> 94 VGPRs) 7.45 -> 7.33 ms, and the RK operands all ahead instead of
-// one variable ahead 7.13 ms (1.78 ms per stage, 3.5 TB/s of HBM traffic);
+// one variable ahead 7.13 ms (112 VGPRs; 1.78 ms per stage, 3.5 TB/s of HBM traffic);
 // three workgroups per CU with two flux buffers (80 VGPRs, five barriers)
 // 7.71 ms.  FP32 tendency (32 x 32 x 16): 90 -> 76 VGPRs, so three workgroups
 // per CU, 1.78 -> 1.63 ms.
